@@ -150,8 +150,9 @@ def median_timed(fn, runs=5, warmup=1):
 
 def cpu_baseline(m, ctx, seconds):
     """Time the CPU oracle decoding from the same synthetic context: one
-    warmup step, then at least 5 timed steps (more while `seconds` lasts);
-    the rate is 1 / the median step time."""
+    warmup step, then at least 5 timed steps (more while `seconds` and the
+    mirror's KV rows last: position n_ctx - 1 is the last one it holds); the
+    rate is 1 / the median step time."""
     import numpy as np
     import oracle
     t0 = time.perf_counter()
@@ -164,7 +165,7 @@ def cpu_baseline(m, ctx, seconds):
         state["pos"] += 1
     step()   # warmup
     ts, spent = [], 0.0
-    while len(ts) < 5 or spent < seconds:
+    while (len(ts) < 5 or spent < seconds) and state["pos"] < m.cfg.n_ctx:
         s = time.perf_counter()
         step()
         ts.append(time.perf_counter() - s)

@@ -1,5 +1,6 @@
 """bench.py's roofline.traffic comes from the committed counter summary only
-while the kernel sources are the ones it was measured on (no GPU)."""
+while the kernel sources are the ones it was measured on, and its CPU
+baseline stays within the positions the model holds (no GPU)."""
 import os
 import sys
 
@@ -23,3 +24,24 @@ def test_traffic_is_null_for_other_sources_or_workloads(monkeypatch):
     assert bench.measured_traffic(16, "q4_k_m", 8192) == (None, None)
     monkeypatch.setattr(bench, "kernel_source_digest", lambda: "0" * 64)
     assert bench.measured_traffic(16, "q4_k_m", 4096) == (None, None)
+
+
+def test_cpu_baseline_stops_at_the_last_kv_row(monkeypatch):
+    """A fast CPU decodes more steps in the time given than the context has
+    rows left; a step past the last row writes past the mirrored KV cache."""
+    import types
+    import oracle
+    seen = []
+
+    class Mirror:
+        def __init__(self, m):
+            pass
+
+        def step(self, tok, pos):
+            seen.append(pos)
+            return tok, None
+
+    monkeypatch.setattr(oracle, "ModelMirror", Mirror)
+    m = types.SimpleNamespace(cfg=types.SimpleNamespace(n_ctx=4157))
+    r = bench.cpu_baseline(m, 4096, 1e9)
+    assert seen == list(range(4096, 4157)) and r["value"] > 0
