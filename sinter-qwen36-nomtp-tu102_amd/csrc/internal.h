@@ -68,6 +68,18 @@ void build_gemv_plan(const sinter_gemv_args &a, uint32_t nblk, GemvPlan &p, uint
 
 namespace sinter {
 
+// the batched GEMV (ubatch.hip): n <= UB_SEGS matrices of one type (Q4_K or
+// Q6_K, nb 256-element items per row) by the same n_tok >= 1 Q8_K activations,
+// one launch; pointers aligned as sinter_op_gemv_ubatch asks
+constexpr uint32_t UB_SEGS = 4;
+struct UbMat {
+    const void *w;
+    float *y;
+    uint32_t rows;
+};
+hipError_t launch_gemv_ubatch(int type, const UbMat *m, uint32_t n, uint32_t nb, const void *xq, uint32_t n_tok,
+                              bool accumulate, hipStream_t s);
+
 // the batched prefill's own kernels (prefill.hip), launched on s
 hipError_t launch_embed_ubatch(const void *embd, int type, uint32_t E, const int32_t *tokens, uint32_t n_tok, float *x,
                                hipStream_t s);

@@ -30,6 +30,8 @@
 #include <cstddef>
 #include <cstring>
 #include <string>
+#include <initializer_list>
+#include <utility>
 #include <vector>
 
 #include "internal.h"
@@ -842,6 +844,18 @@ static int prefill_ubatch(sinter_model *m, uint32_t T, int32_t pos, bool last) {
     auto gemv = [&](const Tensor &w, uint32_t k, float *y, int acc) {
         if (rc == SINTER_OK) rc = sinter_op_gemv_ubatch(w.type, w.d, w.rows, k, p.xq, T, y, acc, sv);
     };
+    // a layer's projections of the same activations: those of one type in one
+    // launch (a 32-row matrix alone would be one workgroup's chain of items)
+    auto gemvs = [&](std::initializer_list<std::pair<const Tensor *, float *>> ms, uint32_t k) {
+        for (int type : {SINTER_Q4_K, SINTER_Q6_K}) {
+            UbMat u[UB_SEGS];
+            uint32_t n = 0;
+            for (const auto &x : ms)
+                if (x.first->type == type) u[n++] = {x.first->d, x.second, (uint32_t)x.first->rows};
+            if (n && rc == SINTER_OK && !hip_ok(launch_gemv_ubatch(type, u, n, k / 256, p.xq, T, false, s), "prefill: projections"))
+                rc = SINTER_ERR_HIP;
+        }
+    };
     auto hip = [&](hipError_t e, const char *what) {
         if (rc == SINTER_OK && !hip_ok(e, what)) rc = SINTER_ERR_HIP;
     };
@@ -851,9 +865,7 @@ static int prefill_ubatch(sinter_model *m, uint32_t T, int32_t pos, bool last) {
         const auto &w = m->W[il];
         rc = sinter_rmsnorm_quant_q8k_ubatch(p.x, (const float *)w[S_ATTN_NORM].d, c.eps, E, T, p.xq, sv);
         if (is_attn(c, il)) {
-            gemv(w[S_WQ], E, p.qg, 0);
-            gemv(w[S_WK], E, p.k, 0);
-            gemv(w[S_WV], E, p.v, 0);
+            gemvs({{&w[S_WQ], p.qg}, {&w[S_WK], p.k}, {&w[S_WV], p.v}}, E);
             hip(launch_attn_prep_ubatch(p.qg, p.k, p.v, (const float *)w[S_Q_NORM].d, (const float *)w[S_K_NORM].d,
                                         m->S[il][0].d, m->S[il][1].d, (uint32_t)c.t_kv, pos, T, NQ, NKV, HD,
                                         (uint32_t)c.rope_dims, theta_scale, c.eps, p.qr, s),
@@ -865,10 +877,7 @@ static int prefill_ubatch(sinter_model *m, uint32_t T, int32_t pos, bool last) {
             if (rc == SINTER_OK) rc = sinter_quant_q8k_ubatch(p.att, (int64_t)NQ * HD, T, p.xq, sv);
             gemv(w[S_WO], NQ * HD, p.x, 1);
         } else {
-            gemv(w[S_QKV], E, p.qkv, 0);
-            gemv(w[S_Z], E, p.z, 0);
-            gemv(w[S_ALPHA], E, p.al, 0);
-            gemv(w[S_BETA], E, p.be, 0);
+            gemvs({{&w[S_QKV], p.qkv}, {&w[S_Z], p.z}, {&w[S_ALPHA], p.al}, {&w[S_BETA], p.be}}, E);
             if (rc == SINTER_OK)
                 rc = sinter_conv_silu_ubatch(p.qkv, (float *)m->S[il][0].d, (const float *)w[S_CONV_W].d, p.conv, C,
                                              (uint32_t)c.conv_k, T, sv);
@@ -883,8 +892,7 @@ static int prefill_ubatch(sinter_model *m, uint32_t T, int32_t pos, bool last) {
         }
         if (rc == SINTER_OK)
             rc = sinter_rmsnorm_quant_q8k_ubatch(p.x, (const float *)w[S_POST_NORM].d, c.eps, E, T, p.xq, sv);
-        gemv(w[S_FFN_GATE], E, p.gate, 0);
-        gemv(w[S_FFN_UP], E, p.up, 0);
+        gemvs({{&w[S_FFN_GATE], p.gate}, {&w[S_FFN_UP], p.up}}, E);
         if (rc == SINTER_OK) rc = sinter_swiglu_quant_q8k_ubatch(p.gate, p.up, F, T, p.xq, sv);
         gemv(w[S_FFN_DOWN], F, p.x, 1);
     }

@@ -7,30 +7,30 @@
 //
 // W: rows x K of ggml Q4_K or Q6_K super-blocks (the GGUF layout as-is);
 // X: n_tokens Q8_K activations (ggml block_q8_K {f32 d; i8 qs[256];
-// i16 bsums[16]}, K/256 blocks per token).  The item terms and their fold
-// are the single-token GEMV's (gemv.h: one fp64 term per 256-element
-// super-block, summed in item order), so every output is bit-identical to
-// the decode GEMV of the same token; only the integer dot products move to
-// MFMA.
+// i16 bsums[16]}, K/256 blocks per token; the sums are taken from the codes).
+// The item terms and their fold are the single-token GEMV's (gemv.h: one fp64
+// term per 256-element super-block, summed in item order), so every output is
+// bit-identical to the decode GEMV of the same token; only the integer dot
+// products move to MFMA.
 //
-// A workgroup of four waves owns 64 rows (16 per wave) and up to 64 tokens
-// (four 16-token tiles), so each weight byte is read from HBM once per 64
-// tokens.  Item by item the workgroup stages the 64 tokens' Q8_K blocks in
-// LDS (double-buffered: the next item's are loaded while this one is
-// computed) and every wave streams its own rows' weights.  Per item
-// and token tile it runs v_mfma_i32_16x16x32_i8 with the tokens' codes as A
-// (16 x 32, lane l: token l%16, elements 8(l/16)..+7 of the 32) and the rows'
-// codes as B (32 x 16, lane l: row l%16, the same elements); D (16 x 16
-// int32, lane l: row l%16, tokens 4(l/16)+v) holds one exact 32-element dot
-// per (token, row).  A Q4_K sub-block is 32 elements, and two of them go
-// through one 64-deep v_mfma_i32_16x16x64_i8 (the pair's 8-byte operands side
-// by side: the sums accumulate over all sub-blocks anyway); a Q6_K sub-block
-// is 16, so a 32-element chunk runs two 32-deep MFMAs, each with the other
-// sub-block's half of B zeroed.  Q4_K's min term sum_s m_s * (sum of the
-// sub-block's activation codes) is one more MFMA per sub-block pair, against
-// B = m_s in every byte, accumulated across the sub-blocks in D.  Each lane then
-// forms the fp64 term of its four (token, row) pairs from its own row's
-// scales and folds it into its accumulators.
+// Both kernels below work on 16 rows x 16 tokens x one item: A = the tokens'
+// codes (lane l: token l%16), B = the rows' codes times their sub-block
+// scales (lane l: row l%16), D (lane l: row l%16, tokens 4(l/16)+v) the item's
+// exact integer sums.  An item takes four 64-deep v_mfma_i32_16x16x64_i8 per
+// digit of code x scale.  Lane group g = l/16 holds 16 consecutive elements
+// of each 64 (WItem::chunk), all of one sub-block: one scale per lane and MFMA.
+//   Q4_K: the 6-bit scale is 8 hi + lo; code x digit (<= 15 * 7) is an int8.
+//     The min term sum_s m_s (sum of sub-block s's codes) is a third MFMA per
+//     chunk, against m_s in every byte.
+//   Q6_K: (code - 32) x scale, at most 4096 in magnitude, is split into
+//     256 h + l with l the signed low byte.
+// Each lane then forms the fp64 terms of its four (token, row) pairs: per
+// pair ((dw * isum) * dx) [- ((dmin * msum) * dx)], equal bit for bit to the
+// decode's (dw * dx) * isum: dw (f16), dx (f32) and the integer leave either
+// first product exact, so both round once, the same exact value.
+#include <algorithm>
+#include <cmath>
+
 #include "internal.h"
 #include "dev_common.h"
 
@@ -38,298 +38,484 @@ namespace sinter {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+typedef double v2d __attribute__((ext_vector_type(2)));
+// 16 bytes at a 4-byte boundary (one global_load_dwordx4)
+typedef struct __attribute__((packed, aligned(4))) { uint32_t d[4]; } u128_a4;
 
-constexpr uint32_t UB_ROWS = 16;     // rows per wave: the MFMA's N
 constexpr uint32_t UB_TOK = 16;      // tokens per tile: the MFMA's M
-constexpr uint32_t UB_TILES = 4;     // token tiles per wave
-constexpr uint32_t UB_TOKENS = UB_TOK * UB_TILES;
-constexpr uint32_t UB_THREADS = 256;  // four waves: 64 rows of the workgroup's row tile
-constexpr uint32_t UB_WG_ROWS = UB_ROWS * (UB_THREADS / 64u);
-constexpr uint32_t UB_XSTRIDE = 68;   // LDS dwords per staged token (65 used)
-// fewest workgroups a launch splits its token groups to reach: two per CU, so
-// each SIMD holds two waves to hide the latency of its MFMA / fp64 chains
-// (4096-token prefill: 1.076 s at one per CU, 1.021 s at 384 or 512, 1.153 s
-// at 768 or 1024, where the 5120-row matrices drop to one token tile per
-// workgroup and read their weights four times)
-constexpr uint64_t UB_MIN_WGS = 512;
+constexpr uint32_t UB_ROWS = 16;     // rows per wave: the MFMA's N
 constexpr uint32_t UB_CONV_MAX = 8;    // conv taps
 constexpr uint32_t Q8K_BYTES = 292;  // block_q8_K
 constexpr uint32_t Q4K_BYTES = 144, Q6K_BYTES = 210;
 
-__device__ __forceinline__ uint32_t ld32(const uint8_t *p) { return *(const uint32_t *)p; }
-__device__ __forceinline__ long pack64(uint32_t lo, uint32_t hi) {
-    return (long)(((unsigned long)hi << 32) | lo);
-}
-// two 8-byte MFMA operands as one 16-byte operand (x in bytes 0-7)
-__device__ __forceinline__ v4i pack128(long x, long y) {
-    const v4i r = {(int)(uint32_t)x, (int)(uint32_t)((unsigned long)x >> 32), (int)(uint32_t)y,
-                   (int)(uint32_t)((unsigned long)y >> 32)};
-    return r;
-}
 __device__ __forceinline__ float f16_bits_to_f32(uint32_t h) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
 }
-// 8 bytes at block byte o of a 2-aligned block whose 4-aligned base is
-// base4 = block - sh (sh = 0 or 2): the third dword is read only when the
-// bytes straddle it, so no read leaves the block's own 4-aligned span
-__device__ __forceinline__ void ld8u(const uint8_t *base4, uint32_t o, uint32_t sh, uint32_t &lo, uint32_t &hi) {
-    const uint32_t *p = (const uint32_t *)(base4 + o);
-    const uint32_t d0 = p[0], d1 = p[1];
-    const uint32_t d2 = sh ? p[2] : 0u;
-    // v_alignbyte_b32: ({d1, d0} >> 8 * sh)[31:0] -- the shift counts bytes
-    lo = __builtin_amdgcn_alignbyte(d1, d0, sh);
-    hi = __builtin_amdgcn_alignbyte(d2, d1, sh);
+// both 16-bit halves of x times s, modulo 2^16 (one v_pk_mul_lo_u16: four
+// byte codes times a digit when no product leaves its byte; a 32-bit multiply
+// would take four times the issue slots)
+__device__ __forceinline__ uint32_t pk_mul(uint32_t x, uint32_t s) {
+    const us2 r = __builtin_bit_cast(us2, x) * (us2)((unsigned short)s);
+    return __builtin_bit_cast(uint32_t, r);
 }
-// bytewise x - 32 for bytes 0..63 (no borrow crosses a byte)
-__device__ __forceinline__ uint32_t sub32b(uint32_t x) { return ((x | 0x80808080u) - 0x20202020u) ^ 0x80808080u; }
+__device__ __forceinline__ uint32_t pk_mad(uint32_t x, uint32_t s, uint32_t c) {
+    const us2 r = __builtin_bit_cast(us2, x) * (us2)((unsigned short)s) + (us2)((unsigned short)c);
+    return __builtin_bit_cast(uint32_t, r);
+}
+
+// One item's MFMA operands of a wave: chunk m of four, the low and high
+// digits of code x scale; the block scales.
+struct BItem {
+    v4i lo[4], hi[4];
+    v4i mn[4];       // Q4_K: the chunk's min in every byte
+    float dw, dmin;
+};
 
 template <int WT>
 struct WItem;
 
-// Q4_K: the lane's row header (d, dmin, 12 scale bytes) and its four 8-byte
-// slices of qs (bytes 32p + 8g..+7: sub-block 2p in the low nibbles, 2p + 1
-// in the high ones)
+// Q4_K.  Chunk m = 2P + n of lane group g: elements 128P + 64(g/2) + 32n +
+// 16(g%2) .. +15 -- n is the nibble, so the lane's two 16-byte loads of qs
+// (at 64P + 16g) serve two chunks each and no byte is loaded twice.
 template <>
 struct WItem<SINTER_Q4_K> {
+    static constexpr uint32_t BYTES = Q4K_BYTES;
+    static constexpr int HI_SHIFT = 3;   // value = lo + (hi << 3)
     uint32_t h[4];
     uint32_t q[8];
-    __device__ __forceinline__ void load(const uint8_t *row, uint32_t i, uint32_t g) {
-        const uint8_t *b = row + (size_t)i * Q4K_BYTES;
+    // the 16-byte chunk (of the item's 16) that lane group g multiplies in MFMA m
+    static __device__ __forceinline__ uint32_t chunk(uint32_t m, uint32_t g) {
+        return 8u * (m >> 1) + 4u * (g >> 1) + 2u * (m & 1u) + (g & 1u);
+    }
+    __device__ __forceinline__ void load(const uint8_t *b, uint32_t g) {
         const uint4 hv = *(const uint4 *)b;
         h[0] = hv.x; h[1] = hv.y; h[2] = hv.z; h[3] = hv.w;
 #pragma unroll
-        for (uint32_t p = 0; p < 4; p++) {
-            const uint2 v = *(const uint2 *)(b + 16u + 32u * p + 8u * g);
-            q[2 * p] = v.x; q[2 * p + 1] = v.y;
+        for (uint32_t P = 0; P < 2; P++) {
+            const uint4 v = *(const uint4 *)(b + 16u + 64u * P + 16u * g);
+            q[4 * P] = v.x; q[4 * P + 1] = v.y; q[4 * P + 2] = v.z; q[4 * P + 3] = v.w;
         }
+    }
+    __device__ __forceinline__ void unpack(BItem &b, uint32_t g) const {
+        // ggml get_scale_min_k4, four sub-blocks at a time; the lane's two
+        // sub-blocks of each half are 2(g/2) and 2(g/2) + 1
+        const uint32_t s0 = h[1], s1 = h[2], s2 = h[3], sh = 16u * (g >> 1);
+        const uint32_t sd[2] = {(s0 & 0x3F3F3F3Fu) >> sh,
+                                ((s2 & 0x0F0F0F0Fu) | ((s0 >> 2) & 0x30303030u)) >> sh};
+        const uint32_t sm[2] = {(s1 & 0x3F3F3F3Fu) >> sh,
+                                (((s2 >> 4) & 0x0F0F0F0Fu) | ((s1 >> 2) & 0x30303030u)) >> sh};
+#pragma unroll
+        for (uint32_t m = 0; m < 4; m++) {
+            const uint32_t P = m >> 1, n = m & 1u;
+            const uint32_t sc = (sd[P] >> (8u * n)) & 0xFFu, dl = sc & 7u, dh = sc >> 3;
+            const int mb = (int)(((sm[P] >> (8u * n)) & 0xFFu) * 0x01010101u);
+            b.mn[m] = v4i{mb, mb, mb, mb};
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++) {
+                const uint32_t c = (q[4 * P + j] >> (4u * n)) & 0x0F0F0F0Fu;
+                b.lo[m][j] = (int)pk_mul(c, dl);
+                b.hi[m][j] = (int)pk_mul(c, dh);
+            }
+        }
+        b.dw = f16_bits_to_f32(h[0] & 0xFFFFu);
+        b.dmin = f16_bits_to_f32(h[0] >> 16);
     }
 };
 
-// Q6_K: the lane's slices of ql (bytes 64n + 8g and 64n + 32 + 8g), qh
-// (bytes 32n + 8g) for both halves n, the 16 int8 scales and d
+// Q6_K.  Chunk m = 2n + k of lane group g: sub-block 8n + 4k + g, elements
+// 128n + 64k + 16g .. +15: the low (k = 0) or high (k = 1) nibbles of the 16
+// bytes ql[64n + 16g ..] and a 2-bit field of the 16 bytes qh[32n + 16(g%2) ..].
 template <>
 struct WItem<SINTER_Q6_K> {
-    uint32_t l0[4], l1[4], hh[4];   // [2n], [2n + 1]: lo / hi dwords of half n
-    uint32_t sc[4];
-    uint32_t d;
-    __device__ __forceinline__ void load(const uint8_t *row, uint32_t i, uint32_t g) {
-        const uint8_t *b = row + (size_t)i * Q6K_BYTES;
-        const uint32_t sh = (uint32_t)((uintptr_t)b & 3u);
-        const uint8_t *b4 = b - sh;
+    static constexpr uint32_t BYTES = Q6K_BYTES;
+    static constexpr int HI_SHIFT = 8;
+    uint32_t l[8], hq[8], sc[5], sh;
+    static __device__ __forceinline__ uint32_t chunk(uint32_t m, uint32_t g) { return 4u * m + g; }
+    // Blocks start on 2-byte boundaries and a 16-byte load that is not
+    // 4-aligned takes four times as long (a wave's load from cache on a busy
+    // CU: 586 cycles at 2 bytes past a boundary, 160 at 4 or 8): each field is
+    // loaded from the 4-aligned address at or before it and shifted into place
+    // with the dword that follows, which is another lane's first (a load of
+    // its own would take as long as the 16 bytes).  No read leaves the
+    // 4-aligned span of the block.
+    __device__ __forceinline__ void load(const uint8_t *b, uint32_t g) {
+        sh = (uint32_t)((uintptr_t)b & 3u);
+        b -= sh;
 #pragma unroll
         for (uint32_t n = 0; n < 2; n++) {
-            ld8u(b4, 64u * n + 8u * g, sh, l0[2 * n], l0[2 * n + 1]);
-            ld8u(b4, 64u * n + 32u + 8u * g, sh, l1[2 * n], l1[2 * n + 1]);
-            ld8u(b4, 128u + 32u * n + 8u * g, sh, hh[2 * n], hh[2 * n + 1]);
+            const uint8_t *p = b + 64u * n + 16u * g, *q = b + 128u + 32u * n + 16u * (g & 1u);
+            const u128_a4 x = *(const u128_a4 *)p, y = *(const u128_a4 *)q;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++) { l[4 * n + j] = x.d[j]; hq[4 * n + j] = y.d[j]; }
         }
-        ld8u(b4, 192u, sh, sc[0], sc[1]);
-        ld8u(b4, 200u, sh, sc[2], sc[3]);
-        d = *(const uint16_t *)(b + 208);
+        const u128_a4 s = *(const u128_a4 *)(b + 192u);   // the scales, then d
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) sc[j] = s.d[j];
+        sc[4] = *(const uint32_t *)(b + 208u);
+    }
+    __device__ __forceinline__ void unpack(BItem &b, uint32_t g) const {
+        const uint32_t f = 2u * (g >> 1);   // the lane's qh field of a nibble: bits f, f + 1 (low), f + 4, f + 5 (high)
+        // the dword after the lane's 16 bytes: the first of lane group g + 1,
+        // and after a field's last group the next field's first
+        const int nl = (int)(4u * ((threadIdx.x + 16u) & 63u));
+        uint32_t ln[2], hn[2];
+#pragma unroll
+        for (uint32_t n = 0; n < 2; n++) {
+            ln[n] = (uint32_t)__builtin_amdgcn_ds_bpermute(nl, (int)(g == 0 ? (n ? hq[0] : l[4]) : l[4 * n]));
+            hn[n] = (uint32_t)__builtin_amdgcn_ds_bpermute(nl, (int)((g & 1u) == 0 ? (n ? sc[0] : hq[4]) : hq[4 * n]));
+        }
+#pragma unroll
+        for (uint32_t n = 0; n < 2; n++) {
+            uint32_t s[2], bias[2];
+#pragma unroll
+            for (uint32_t k = 0; k < 2; k++) {
+                // sub-block 4 (2n + k) + g's signed scale, 16 bits (mod 2^16 arithmetic)
+                const uint32_t w = __builtin_amdgcn_alignbyte(sc[2 * n + k + 1], sc[2 * n + k], sh);
+                s[k] = (uint32_t)(int)(int8_t)((w >> (8u * g)) & 0xFFu) & 0xFFFFu;
+                bias[k] = 128u - 32u * s[k];
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++) {
+                const uint32_t lw = __builtin_amdgcn_alignbyte(j < 3 ? l[4 * n + j + 1] : ln[n], l[4 * n + j], sh);
+                const uint32_t hw = __builtin_amdgcn_alignbyte(j < 3 ? hq[4 * n + j + 1] : hn[n], hq[4 * n + j], sh) >> f;
+#pragma unroll
+                for (uint32_t k = 0; k < 2; k++) {
+                    const uint32_t m = 2 * n + k;
+                    // code + 32, 0..63
+                    const uint32_t u = ((lw >> (4u * k)) & 0x0F0F0F0Fu) | ((k ? hw : hw << 4) & 0x30303030u);
+                    // p + 128 of the even and odd bytes, p = (u - 32) * scale:
+                    // the high byte of p + 128 is h, its low byte l + 128
+                    const uint32_t pe = pk_mad(u & 0x00FF00FFu, s[k], bias[k]);
+                    const uint32_t po = pk_mad((u >> 8) & 0x00FF00FFu, s[k], bias[k]);
+                    b.lo[m][j] = (int)(__builtin_amdgcn_perm(po, pe, 0x06020400u) ^ 0x80808080u);
+                    b.hi[m][j] = (int)__builtin_amdgcn_perm(po, pe, 0x07030501u);
+                }
+            }
+        }
+        const uint32_t d = (sc[4] >> (8u * sh)) & 0xFFFFu;
+        b.dw = f16_bits_to_f32(d);
+        b.dmin = 0.0f;
     }
 };
 
-// Stage item i of the workgroup's tokens in LDS: token j's Q8_K block i (its
-// 256 codes at dwords 0..63 of LDS row j, its d at dword 64).  Wave w stages
-// token tile w, four lanes per token, each lane 16 code dwords (and the
-// first of the four, d), so the per-item work is one address update and
-// loads at immediate offsets.  Tokens past the last repeat it (never
-// stored).  ld: into registers; st: registers to LDS buffer xs.
-struct ActStage {
-    uint32_t v[16], d;
-    const uint8_t *blk0;   // the lane's token's block 0
-    uint32_t part, row;    // 16-dword quarter of the codes; LDS row (token within the group)
-    __device__ __forceinline__ void init(const uint8_t *xq, uint32_t nb, uint32_t tok0, uint32_t n_tok) {
-        const uint32_t lane = threadIdx.x & 63u;
-        row = UB_TOK * (threadIdx.x >> 6) + (lane >> 2);
-        part = lane & 3u;
-        const uint32_t tok = min(tok0 + row, n_tok - 1u);
-        blk0 = xq + (size_t)tok * nb * Q8K_BYTES;
-    }
-    __device__ __forceinline__ void ld(uint32_t i) {
-        const uint8_t *b = blk0 + (size_t)i * Q8K_BYTES;
-        const uint32_t *c = (const uint32_t *)(b + 4u + 64u * part);
-#pragma unroll
-        for (uint32_t k = 0; k < 16; k++) v[k] = c[k];
-        if (part == 0) d = *(const uint32_t *)b;
-    }
-    __device__ __forceinline__ void st(uint32_t *xs) const {
-        uint32_t *r = xs + row * UB_XSTRIDE;
-#pragma unroll
-        for (uint32_t k = 0; k < 4; k++)
-            *(uint4 *)(r + 16u * part + 4u * k) = make_uint4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
-        if (part == 0) r[64] = d;
-    }
+// The exact integer sums of one tile: lo / hi digits and (Q4_K) the min sums.
+struct Sums {
+    v4i lo, hi, mn;
 };
-static_assert(UB_THREADS / 64u == UB_TILES, "one staging wave per token tile");
-static_assert(UB_XSTRIDE % 4u == 0, "16-byte LDS row alignment");
-
 template <int WT>
-__global__ __launch_bounds__(UB_THREADS) void ubatch_gemv_kernel(const uint8_t *__restrict__ w, uint32_t rows,
-                                                                uint32_t nb, const uint8_t *__restrict__ xq,
-                                                                uint32_t n_tok, float *__restrict__ y, uint32_t n_tg,
-                                                                uint32_t tpw, uint32_t accumulate) {
-    __shared__ uint32_t xs[2][UB_TOKENS * UB_XSTRIDE];
-    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6, r = lane & 15u, g = lane >> 4;
-    // adjacent workgroups share a row tile (their token groups): its weight
-    // bytes come from HBM once and from the memory-side cache after
-    const uint32_t rt = blockIdx.x / n_tg, tg = blockIdx.x % n_tg;
-    const uint32_t row = rt * UB_WG_ROWS + wv * UB_ROWS + r;
-    const uint32_t rowc = row < rows ? row : rows - 1u;
-    const uint32_t tok0 = tg * UB_TOK * tpw;
-    const uint32_t ntiles = min(tpw, (n_tok - tok0 + UB_TOK - 1u) / UB_TOK);   // block-uniform, 1..4
-    const size_t row_bytes = (size_t)nb * (WT == SINTER_Q4_K ? Q4K_BYTES : Q6K_BYTES);
-    const uint8_t *wrow = w + (size_t)rowc * row_bytes;
-
-    double acc[UB_TILES][4];
+__device__ __forceinline__ Sums tile_sums(const v4i a[4], const BItem &b) {
+    const v4i z = {0, 0, 0, 0};
+    Sums s = {z, z, z};
 #pragma unroll
-    for (uint32_t t = 0; t < UB_TILES; t++)
+    for (uint32_t m = 0; m < 4; m++) {
+        s.lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[m], b.lo[m], s.lo, 0, 0, 0);
+        s.hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[m], b.hi[m], s.hi, 0, 0, 0);
+        if constexpr (WT == SINTER_Q4_K) s.mn = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[m], b.mn[m], s.mn, 0, 0, 0);
+    }
+    return s;
+}
+// the fp64 terms of the lane's four pairs
+template <int WT>
+__device__ __forceinline__ void tile_terms(const Sums &s, double dw, double dmin, const double dx[4], double t[4]) {
+    double p[4], q[4];
+#pragma unroll
+    for (uint32_t v = 0; v < 4; v++)
+        p[v] = (double)(int)((uint32_t)s.lo[v] + ((uint32_t)s.hi[v] << WItem<WT>::HI_SHIFT));
+    if constexpr (WT == SINTER_Q4_K) {
+#pragma unroll
+        for (uint32_t v = 0; v < 4; v++) q[v] = (double)s.mn[v];
+    }
+#pragma unroll
+    for (uint32_t v = 0; v < 4; v++) p[v] = (dw * p[v]) * dx[v];
+    if constexpr (WT == SINTER_Q4_K) {
+#pragma unroll
+        for (uint32_t v = 0; v < 4; v++) q[v] = (dmin * q[v]) * dx[v];
+#pragma unroll
+        for (uint32_t v = 0; v < 4; v++) p[v] = p[v] - q[v];
+    }
+#pragma unroll
+    for (uint32_t v = 0; v < 4; v++) t[v] = p[v];
+}
+
+// One launch multiplies up to UB_SEGS matrices of one type by the same
+// activations (a layer's projections): row tiles of all of them in one grid.
+struct UbArgs {
+    const uint8_t *xq;
+    uint32_t nb, n_tok, n_tg, accumulate, n_seg;
+    uint32_t rt0[UB_SEGS];     // first row tile of each matrix
+    uint32_t rows[UB_SEGS];
+    const uint8_t *w[UB_SEGS];
+    float *y[UB_SEGS];
+};
+// workgroup -> (row tile, token group): workgroups are dealt to the 8 XCDs in
+// turn, so XCD x takes the x-th eighth of the tiles and the token groups of
+// one row tile (which read the same weights) share its L2
+__device__ __forceinline__ void ub_tile(const UbArgs &a, uint32_t &rt, uint32_t &tg) {
+    const uint32_t n = gridDim.x, x = blockIdx.x & 7u, q = n >> 3, r = n & 7u;
+    const uint32_t id = x * q + min(x, r) + (blockIdx.x >> 3);
+    rt = id / a.n_tg;
+    tg = id % a.n_tg;
+}
+
+// ---------------------------------------------------------------- many tokens
+
+// A workgroup of four waves owns 64 rows (16 per wave) and NT token tiles.
+// Per item the tokens' codes arrive in LDS by LDS-DMA (double-buffered, one
+// item ahead) and each wave unpacks its rows' weights (in registers, two items
+// ahead) once for its NT tiles.  A token's 256 codes are 16 chunks of 16
+// bytes; chunk c of token r lies in slot c ^ (r % 16), so the 16 tokens' reads
+// of one chunk fall on distinct banks without padding, which the DMA's
+// contiguous kilobyte per wave could not leave.
+constexpr uint32_t UB_THREADS = 256;
+constexpr uint32_t UB_WG_ROWS = UB_ROWS * (UB_THREADS / 64u);
+constexpr uint32_t UB_TILE_BYTES = UB_TOK * 256u;
+// a buffer: codes | dx f64 [token]
+template <uint32_t NT>
+constexpr uint32_t ub_buf() { return NT * (UB_TILE_BYTES + UB_TOK * 8u); }
+// the DMA's 32-bit lane offsets reach 128 tokens of items
+constexpr uint32_t UB_MAX_NB = 50000;
+
+template <int WT, uint32_t NT>
+__global__ __launch_bounds__(UB_THREADS, 2) void ubatch_gemm_kernel(UbArgs a) {
+    __shared__ __attribute__((aligned(16))) unsigned char xs[2 * ub_buf<NT>()];
+    LDS unsigned char *L = (LDS unsigned char *)xs;
+    const uint32_t lbase = (uint32_t)(uintptr_t)L;
+    const uint32_t lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t r = lane & 15u, g = lane >> 4;
+    uint32_t rt, tg;
+    ub_tile(a, rt, tg);
+    uint32_t sg = 0;
+    while (sg + 1u < a.n_seg && rt >= a.rt0[sg + 1u]) sg++;
+    const uint32_t rows = a.rows[sg], nb = a.nb, n_tok = a.n_tok;
+    const uint32_t row = (rt - a.rt0[sg]) * UB_WG_ROWS + wv * UB_ROWS + r;
+    const uint32_t tok0 = tg * UB_TOK * NT, tl = n_tok - 1u - tok0;   // (tokens past the last repeat it, never stored)
+    const uint8_t *wp = a.w[sg] + (size_t)min(row, rows - 1u) * nb * WItem<WT>::BYTES;
+    const uint8_t *xp = a.xq + (size_t)tok0 * nb * Q8K_BYTES;   // (uniform)
+    // DMA j of wave w fills tokens 16 j + 4 w .. + 3: lane l token l / 16 of
+    // them, slot l % 16
+    uint32_t xo[NT];
+#pragma unroll
+    for (uint32_t j = 0; j < NT; j++) {
+        const uint32_t tk = 4u * wv + g;
+        xo[j] = min(UB_TOK * j + tk, tl) * nb * Q8K_BYTES + 4u + 16u * (r ^ tk);
+    }
+    const uint32_t dxo = min(min(threadIdx.x, UB_TOK * NT - 1u), tl) * nb * Q8K_BYTES;
+    uint32_t ao[4];   // the lane's four chunks of tile 0
+#pragma unroll
+    for (uint32_t m = 0; m < 4; m++) ao[m] = r * 256u + 16u * (WItem<WT>::chunk(m, g) ^ r);
+
+    double acc[NT][4];
+#pragma unroll
+    for (uint32_t t = 0; t < NT; t++)
 #pragma unroll
         for (uint32_t v = 0; v < 4; v++) acc[t][v] = 0.0;
 
-    ActStage stage;
-    // wave w stages token tile w, when the group has it (wave-uniform)
-    const bool stager = (threadIdx.x >> 6) < ntiles;
-    stage.init(xq, nb, tok0, n_tok);
-    if (stager) stage.ld(0);
-    WItem<WT> cur, nxt;
-    cur.load(wrow, 0, g);
-    if (stager) stage.st(xs[0]);
-    __syncthreads();
-    for (uint32_t i = 0; i < nb; i++) {
-        if (i + 1u < nb) {
-            // activations first: vector loads complete in order, so the
-            // staging store at the end of this item then waits for these
-            // cache hits and not for the weights behind them
-            if (stager) stage.ld(i + 1u);
-            nxt.load(wrow, i + 1u, g);
-        }
-        const uint32_t *xb = xs[i & 1u];
-
-        // B operands and the per-sub-block integer scales of the lane's row
-        long b[8];       // Q4_K: codes x the scale's low 3 bits; Q6_K: codes
-        long bh[8];      // Q4_K: codes x the scale's high 3 bits
-        long bm[8];      // Q4_K: the min in every byte
-        int scl[16];     // Q6_K: the 16 sub-block scales
-        float dw, dmin = 0.0f;
-        if constexpr (WT == SINTER_Q4_K) {
-            // ggml get_scale_min_k4 for sub-blocks 0..7, four at a time
-            const uint32_t s0 = cur.h[1], s1 = cur.h[2], s2 = cur.h[3];
-            const uint32_t dlo = s0 & 0x3F3F3F3Fu, mlo = s1 & 0x3F3F3F3Fu;
-            const uint32_t dhi = (s2 & 0x0F0F0F0Fu) | ((s0 >> 2) & 0x30303030u);
-            const uint32_t mhi = ((s2 >> 4) & 0x0F0F0F0Fu) | ((s1 >> 2) & 0x30303030u);
+    float dxn = 0.0f;
+    auto stage = [&](uint32_t i, uint32_t buf) {
+        const uint8_t *q = xp + (size_t)i * Q8K_BYTES;
+        const uintptr_t p = (uintptr_t)q;
 #pragma unroll
-            for (uint32_t s = 0; s < 8; s++) {
-                const uint32_t sd = ((s < 4 ? dlo : dhi) >> (8u * (s & 3u))) & 0xFFu;
-                const uint32_t sm = ((s < 4 ? mlo : mhi) >> (8u * (s & 3u))) & 0xFFu;
-                const uint32_t mm = sm * 0x01010101u;
-                bm[s] = pack64(mm, mm);
-                const uint32_t p = s >> 1, sh = 4u * (s & 1u);
-                const uint32_t q0 = (cur.q[2 * p] >> sh) & 0x0F0F0F0Fu, q1 = (cur.q[2 * p + 1] >> sh) & 0x0F0F0F0Fu;
-                // scale = 8 hi + lo (hi, lo <= 7): a code (<= 15) times either
-                // fits a byte (<= 105), so one 32-bit multiply scales four
-                // codes with no carry between them, and the products are
-                // int8 operands
-                const uint32_t lo = sd & 7u, hi = sd >> 3;
-                b[s] = pack64(q0 * lo, q1 * lo);
-                bh[s] = pack64(q0 * hi, q1 * hi);
+        for (uint32_t j = 0; j < NT; j++)
+            lds_dma16<false>(p, xo[j], lbase + buf * ub_buf<NT>() + j * UB_TILE_BYTES + wv * 1024u);
+        dxn = *(const float *)(q + dxo);
+    };
+    auto park = [&](uint32_t buf) {
+        if (threadIdx.x < UB_TOK * NT)
+            *reinterpret_cast<LDS double *>(L + buf * ub_buf<NT>() + NT * UB_TILE_BYTES + 8u * threadIdx.x) = (double)dxn;
+    };
+    struct AFrag { v4i x[4]; v2d d0, d1; };
+    // item i: its codes in buffer `buf`, its weights in w
+    auto item = [&](uint32_t i, uint32_t buf, WItem<WT> &w) {
+        const LDS unsigned char *xb = L + buf * ub_buf<NT>(), *dxs = xb + NT * UB_TILE_BYTES + 32u * g;
+        auto lda = [&](uint32_t t) {
+            AFrag f;
+#pragma unroll
+            for (uint32_t m = 0; m < 4; m++) f.x[m] = *reinterpret_cast<const LDS v4i *>(xb + ao[m] + t * UB_TILE_BYTES);
+            const LDS v2d *q = reinterpret_cast<const LDS v2d *>(dxs + t * UB_TOK * 8u);
+            f.d0 = q[0];
+            f.d1 = q[1];
+            return f;
+        };
+        // (the empty asm statements keep the compiler from sinking the
+        // arithmetic past the loads that it is to run beside, or past the
+        // barrier: the unpacking would wait for the loads behind it)
+        BItem b;
+        w.unpack(b, g);
+#pragma unroll
+        for (uint32_t m = 0; m < 4; m++) {
+            asm volatile("" : "+v"(b.lo[m]), "+v"(b.hi[m]));
+            if constexpr (WT == SINTER_Q4_K) asm volatile("" : "+v"(b.mn[m]));
+        }
+        sched_fence();
+        // the next item's activations, then the weights of the one after it:
+        // loads complete in order, so the wait below leaves the weights in
+        // flight (past the end: the last item again, never used)
+        stage(min(i + 1u, nb - 1u), buf ^ 1u);
+        sched_fence();
+        w.load(wp + (size_t)min(i + 2u, nb - 1u) * WItem<WT>::BYTES, g);
+        AFrag f = lda(0), fn;
+        sched_fence();
+        const double dw = (double)b.dw, dmin = (double)b.dmin;
+        // tile t's MFMAs run beside tile t - 1's fp64 terms and tile t + 1's reads
+        Sums s, sp;
+        double dxp[4];
+#pragma unroll
+        for (uint32_t t = 0; t <= NT; t++) {
+            if (t + 1 < NT) fn = lda(t + 1);
+            sched_fence();
+            if (t < NT) s = tile_sums<WT>(f.x, b);
+            if (t > 0) {
+                double tm[4];
+                tile_terms<WT>(sp, dw, dmin, dxp, tm);
+#pragma unroll
+                for (uint32_t v = 0; v < 4; v++) acc[t - 1][v] += tm[v];
+                asm volatile("" : "+v"(acc[t - 1][0]), "+v"(acc[t - 1][1]), "+v"(acc[t - 1][2]), "+v"(acc[t - 1][3]));
             }
-            dw = f16_bits_to_f32(cur.h[0] & 0xFFFFu);
-            dmin = f16_bits_to_f32(cur.h[0] >> 16);
-        } else {
-#pragma unroll
-            for (uint32_t c = 0; c < 8; c++) {
-                const uint32_t n = c >> 2, q = c & 3u;
-                const uint32_t *L = (q & 1u) ? cur.l1 : cur.l0;
-                const uint32_t ls = 4u * (q >> 1), hs = 2u * q;
-                uint32_t lo = ((L[2 * n] >> ls) & 0x0F0F0F0Fu) | (((cur.hh[2 * n] >> hs) & 0x03030303u) << 4);
-                uint32_t hi = ((L[2 * n + 1] >> ls) & 0x0F0F0F0Fu) | (((cur.hh[2 * n + 1] >> hs) & 0x03030303u) << 4);
-                b[c] = pack64(sub32b(lo), sub32b(hi));
+            if (t < NT) asm volatile("" : "+v"(s.lo), "+v"(s.hi));
+            sched_fence();
+            if (t < NT) {
+                sp = s;
+                dxp[0] = f.d0[0]; dxp[1] = f.d0[1]; dxp[2] = f.d1[0]; dxp[3] = f.d1[1];
             }
-#pragma unroll
-            for (uint32_t j = 0; j < 16; j++) scl[j] = (int)(int8_t)((cur.sc[j >> 2] >> (8u * (j & 3u))) & 0xFFu);
-            dw = f16_bits_to_f32(cur.d);
+            f = fn;
         }
-
-#pragma unroll
-        for (uint32_t t = 0; t < UB_TILES; t++) {
-            if (t < ntiles) {
-                // A: token 16t + r, elements 32c + 8g..+7 (row stride 68 dwords: the
-                // 32 lanes of a half-wave read 32 distinct bank pairs)
-                const uint32_t *xa = xb + (UB_TOK * t + r) * UB_XSTRIDE + 2u * g;
-                long a[8];
-#pragma unroll
-                for (uint32_t c = 0; c < 8; c++) {
-                    const uint2 v2 = *(const uint2 *)(xa + 8u * c);
-                    a[c] = pack64(v2.x, v2.y);
-                }
-                float dx[4];
-#pragma unroll
-                for (uint32_t v = 0; v < 4; v++)
-                    dx[v] = __builtin_bit_cast(float, xb[(UB_TOK * t + 4u * g + v) * UB_XSTRIDE + 64u]);
-                const v4i z = {0, 0, 0, 0};
-                int isum[4] = {0, 0, 0, 0};
-                if constexpr (WT == SINTER_Q4_K) {
-                    // sum_s scale_s dot_s = 8 sum_s hi_s dot_s + sum_s lo_s dot_s, all
-                    // exact in int32 (|each| <= 256 * 105 * 128).  Sub-blocks s and
-                    // s + 1 go through one 64-deep MFMA: A and B carry sub-block s in
-                    // bytes 0-7 of each lane and s + 1 in bytes 8-15 (the MFMA pairs
-                    // A and B bytes by the same lane-group / byte k index, so any
-                    // common placement gives the same exact sums)
-                    v4i cm = z, ch = z, cl = z;
-#pragma unroll
-                    for (uint32_t s = 0; s < 8; s += 2) {
-                        const v4i a2 = pack128(a[s], a[s + 1]);
-                        cl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, pack128(b[s], b[s + 1]), cl, 0, 0, 0);
-                        ch = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, pack128(bh[s], bh[s + 1]), ch, 0, 0, 0);
-                        cm = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, pack128(bm[s], bm[s + 1]), cm, 0, 0, 0);
-                    }
-#pragma unroll
-                    for (uint32_t v = 0; v < 4; v++) {
-                        isum[v] = 8 * ch[v] + cl[v];
-                        const double dxd = (double)dx[v];
-                        const double t1 = ((double)dw * dxd) * (double)isum[v];
-                        const double t2 = ((double)dmin * dxd) * (double)cm[v];
-                        acc[t][v] += t1 - t2;
-                    }
-                } else {
-                    const bool lo_half = g < 2u;
-#pragma unroll
-                    for (uint32_t c = 0; c < 8; c++) {
-                        const long b0 = lo_half ? b[c] : 0l, b1 = lo_half ? 0l : b[c];
-                        const v4i c0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a[c], b0, z, 0, 0, 0);
-                        const v4i c1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a[c], b1, z, 0, 0, 0);
-                        // |scale| <= 128, |dot| <= 16 * 32 * 128: 24-bit products
-#pragma unroll
-                        for (uint32_t v = 0; v < 4; v++)
-                            isum[v] += __mul24(scl[2 * c], c0[v]) + __mul24(scl[2 * c + 1], c1[v]);
-                    }
-#pragma unroll
-                    for (uint32_t v = 0; v < 4; v++) acc[t][v] += ((double)dw * (double)dx[v]) * (double)isum[v];
-                }
-            }
-        }
-        if (i + 1u < nb) {
-            cur = nxt;
-            // buffer (i + 1) & 1 was last read for item i - 1, before the
-            // barrier that ended that item
-            if (stager) stage.st(xs[(i + 1u) & 1u]);
-        }
+        // every wave waits for dxn, which it loaded after its share of the
+        // DMAs: loads complete in order, so they have landed (the weights
+        // behind them may still fly)
+        asm volatile("" : "+v"(dxn)::"memory");
+        park(buf ^ 1u);
         __syncthreads();
+    };
+    WItem<WT> w0, w1;
+    stage(0, 0);
+    sched_fence();
+    w0.load(wp, g);
+    w1.load(wp + (size_t)min(1u, nb - 1u) * WItem<WT>::BYTES, g);
+    park(0);
+    dma_wait();
+    __syncthreads();
+    for (uint32_t i = 0; i < nb; i += 2) {
+        item(i, 0, w0);
+        if (i + 1u < nb) item(i + 1u, 1, w1);
     }
+    dma_wait();   // (the last item's staging must not outlive the workgroup's LDS)
 
     if (row < rows) {
+        float *y = a.y[sg] + row;
 #pragma unroll
-        for (uint32_t t = 0; t < UB_TILES; t++)
+        for (uint32_t t = 0; t < NT; t++)
 #pragma unroll
             for (uint32_t v = 0; v < 4; v++) {
                 const uint32_t tok = tok0 + t * UB_TOK + 4u * g + v;
-                if (t < ntiles && tok < n_tok) {
+                if (tok < n_tok) {
                     // accumulate: the residual add of the single-token GEMV's
                     // RESID epilogue (y = y + result, one fp32 add)
-                    float *yp = y + (size_t)tok * rows + row;
-                    *yp = accumulate ? *yp + (float)acc[t][v] : (float)acc[t][v];
+                    float *yp = y + (size_t)tok * rows;
+                    *yp = a.accumulate ? *yp + (float)acc[t][v] : (float)acc[t][v];
                 }
             }
+    }
+}
+
+// ---------------------------------------------------------------- few tokens
+
+// With few tokens the weights bound the time: a workgroup owns 16 rows and NT
+// token tiles, and its KW waves take the items in turn (wave w items w, w +
+// KW, ...), each wave's weights and activations straight from memory, so the
+// loads of a whole row are in flight at once.  The terms of a round of KW
+// items meet in LDS (double-buffered), where each (row, token) is folded by
+// one thread in item order.
+constexpr uint32_t UB_KW = 4;
+template <int WT, uint32_t NT>
+__global__ __launch_bounds__(64 * UB_KW) void ubatch_gemv_kernel(UbArgs a) {
+    constexpr uint32_t KW = UB_KW, OUT = NT * UB_TOK * UB_ROWS, THREADS = 64u * KW, PT = (OUT + THREADS - 1u) / THREADS;
+    __shared__ double terms[2][KW][OUT];
+    LDS double *T = (LDS double *)terms;
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6, r = lane & 15u, g = lane >> 4;
+    uint32_t rt, tg;
+    ub_tile(a, rt, tg);
+    uint32_t sg = 0;
+    while (sg + 1u < a.n_seg && rt >= a.rt0[sg + 1u]) sg++;
+    const uint32_t rows = a.rows[sg], nb = a.nb, n_tok = a.n_tok;
+    const uint32_t row0 = (rt - a.rt0[sg]) * UB_ROWS, tok0 = tg * UB_TOK * NT;
+    const uint8_t *wrow = a.w[sg] + (size_t)min(row0 + r, rows - 1u) * nb * WItem<WT>::BYTES;
+    const uint8_t *xrow[NT], *drow[NT][4];
+#pragma unroll
+    for (uint32_t t = 0; t < NT; t++) {   // (tokens past the last repeat it, never stored)
+        xrow[t] = a.xq + (size_t)min(tok0 + UB_TOK * t + r, n_tok - 1u) * nb * Q8K_BYTES;
+#pragma unroll
+        for (uint32_t v = 0; v < 4; v++)
+            drow[t][v] = a.xq + (size_t)min(tok0 + UB_TOK * t + 4u * g + v, n_tok - 1u) * nb * Q8K_BYTES;
+    }
+    double acc[PT];
+#pragma unroll
+    for (uint32_t p = 0; p < PT; p++) acc[p] = 0.0;
+    const uint32_t rounds = (nb + KW - 1u) / KW;
+    struct XItem { v4i x[NT][4]; float dx[NT][4]; };
+    WItem<WT> w;
+    auto load_x = [&](XItem &X, uint32_t i) {
+#pragma unroll
+        for (uint32_t t = 0; t < NT; t++) {
+#pragma unroll
+            for (uint32_t m = 0; m < 4; m++) {
+                const u128_a4 c = *(const u128_a4 *)(xrow[t] + (size_t)i * Q8K_BYTES + 4u + 16u * WItem<WT>::chunk(m, g));
+                X.x[t][m] = v4i{(int)c.d[0], (int)c.d[1], (int)c.d[2], (int)c.d[3]};
+            }
+#pragma unroll
+            for (uint32_t v = 0; v < 4; v++) X.dx[t][v] = *(const float *)(drow[t][v] + (size_t)i * Q8K_BYTES);
+        }
+    };
+    // round q: this wave's item from X, the next round's loads (into w and
+    // Xn) in flight behind its arithmetic, the terms folded
+    auto round = [&](uint32_t q, const XItem &X, XItem &Xn) {
+        const uint32_t i = q * KW + wv;   // (items past the last repeat it, their terms never folded)
+        BItem b;
+        w.unpack(b, g);
+        __builtin_amdgcn_sched_barrier(0);
+        if (q + 1u < rounds) {
+            const uint32_t in = min(i + KW, nb - 1u);
+            w.load(wrow + (size_t)in * WItem<WT>::BYTES, g);
+            load_x(Xn, in);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const double dw = (double)b.dw, dmin = (double)b.dmin;
+        LDS double *Tb = T + (q & 1u) * KW * OUT;
+#pragma unroll
+        for (uint32_t t = 0; t < NT; t++) {
+            const Sums u = tile_sums<WT>(X.x[t], b);
+            const double dx[4] = {(double)X.dx[t][0], (double)X.dx[t][1], (double)X.dx[t][2], (double)X.dx[t][3]};
+            double tm[4];
+            tile_terms<WT>(u, dw, dmin, dx, tm);
+#pragma unroll
+            for (uint32_t v = 0; v < 4; v++) Tb[wv * OUT + (UB_TOK * t + 4u * g + v) * UB_ROWS + r] = tm[v];
+        }
+        __syncthreads();   // (the other buffer's readers are past it: they wrote their terms after reading)
+        const uint32_t n = min(KW, nb - q * KW);
+#pragma unroll
+        for (uint32_t p = 0; p < PT; p++) {
+            const uint32_t o = threadIdx.x + p * THREADS;
+            if (OUT % THREADS == 0 || o < OUT) {
+#pragma unroll
+                for (uint32_t k = 0; k < KW; k++)
+                    if (k < n) acc[p] += Tb[k * OUT + o];
+            }
+        }
+    };
+    XItem X0, X1;
+    w.load(wrow + (size_t)min(wv, nb - 1u) * WItem<WT>::BYTES, g);
+    load_x(X0, min(wv, nb - 1u));
+    for (uint32_t q = 0; q < rounds; q += 2) {
+        round(q, X0, X1);
+        if (q + 1u < rounds) round(q + 1u, X1, X0);
+    }
+#pragma unroll
+    for (uint32_t p = 0; p < PT; p++) {
+        const uint32_t o = threadIdx.x + p * THREADS, tok = tok0 + o / UB_ROWS, row = row0 + o % UB_ROWS;
+        if (o < OUT && tok < n_tok && row < rows) {
+            float *yp = a.y[sg] + (size_t)tok * rows + row;
+            *yp = a.accumulate ? *yp + (float)acc[p] : (float)acc[p];
+        }
     }
 }
 
@@ -534,6 +720,117 @@ __global__ __launch_bounds__(256) void rmsnorm_quant_q8k_kernel(const float *__r
 
 using namespace sinter;
 
+namespace sinter {
+namespace {
+
+// The split of a launch: token tiles per workgroup, few-token or many-token kernel.
+struct UbSplit {
+    bool few;
+    uint32_t nt, wg_rows, n_tg;
+    uint64_t wgs;
+};
+
+// The cheapest of the compiled splits by a cost per item, fitted to times of
+// 11 matrices (32..34816 rows, K 4096..17408) x 10 token counts (8..512); ns:
+//   many-token kernel: up to one workgroup per CU it runs at its latency
+//   `lone`; with w > 1 per CU the CU's issue slots bound it, `thr` per
+//   workgroup, and a started last round takes about two thirds of one;
+//   few-token kernel: latency, or `thr` per workgroup of a CU over a start-up.
+// E.g. Q6_K 5120 x 17408 at 256 tokens (us): nt 2 180, 3 131, 4 143, 6 118,
+// 8 143; at 8 tokens few-token 39, many-token 86.  Q4_K 34816 x 5120 at 256:
+// nt 2 205, 4 180, 6 181, 8 166; 8192 x 5120 at 24: few-token 15, nt 1 15.5.
+template <int WT>
+UbSplit ub_split(const UbArgs &a) {
+    constexpr bool Q4 = WT == SINTER_Q4_K;
+    const uint32_t tiles = (a.n_tok + UB_TOK - 1) / UB_TOK;
+    UbSplit best = {};
+    double cost = 1e300;
+    auto consider = [&](bool few, uint32_t nt, double lone, double thr, double start) {
+        UbSplit s;
+        s.few = few;
+        s.nt = nt;
+        s.wg_rows = few ? UB_ROWS : UB_WG_ROWS;
+        s.n_tg = (tiles + nt - 1) / nt;
+        uint64_t n_rt = 0;
+        for (uint32_t i = 0; i < a.n_seg; i++) n_rt += ((uint64_t)a.rows[i] + s.wg_rows - 1) / s.wg_rows;
+        s.wgs = n_rt * s.n_tg;
+        const double w = (double)s.wgs / 256.0;
+        double c;
+        if (few) c = std::max(lone, start + w * thr);
+        else c = start + (w <= 1.0 ? lone : std::max(lone, std::floor(w) * thr) + (w > std::floor(w) ? 0.65 * thr : 0.0));
+        if (c < cost) { cost = c; best = s; }
+    };
+    // (not compiled, as never the cheapest: few-token nt 2 for Q4_K, whose
+    // unpacking is cheap enough to repeat; many-token nt 1 for Q6_K, whose is not)
+    consider(true, 1, Q4 ? 370 : 560, Q4 ? 166 : 250, Q4 ? 200 : 150);
+    if (!Q4 && tiles > 1) consider(true, 2, 700, 420, 150);
+    if (a.nb > UB_MAX_NB) return best;
+    for (uint32_t nt : {Q4 ? 1u : 2u, 2u, 3u, 4u, 6u, 8u})
+        consider(false, nt, Q4 ? 477 + 168 * nt : 1030 + 108 * nt, Q4 ? 190 + 215 * nt : 550 + 150 * nt, 125);
+    return best;
+}
+
+template <int WT, uint32_t NT>
+void launch_gemm(const UbArgs &a, uint32_t grid, hipStream_t s) {
+    hipLaunchKernelGGL((ubatch_gemm_kernel<WT, NT>), dim3(grid), dim3(UB_THREADS), 0, s, a);
+}
+template <int WT, uint32_t NT>
+void launch_gemv(const UbArgs &a, uint32_t grid, hipStream_t s) {
+    hipLaunchKernelGGL((ubatch_gemv_kernel<WT, NT>), dim3(grid), dim3(64 * UB_KW), 0, s, a);
+}
+
+template <int WT>
+hipError_t launch_ubatch(UbArgs &a, hipStream_t s) {
+    const UbSplit p = ub_split<WT>(a);
+    if (p.wgs > (uint64_t)INT32_MAX) return hipErrorInvalidValue;
+    a.n_tg = p.n_tg;
+    uint32_t n_rt = 0;
+    for (uint32_t i = 0; i < a.n_seg; i++) {
+        a.rt0[i] = n_rt;
+        n_rt += (uint32_t)(((uint64_t)a.rows[i] + p.wg_rows - 1) / p.wg_rows);
+    }
+    const uint32_t grid = (uint32_t)p.wgs;
+    if (p.few) {
+        if constexpr (WT == SINTER_Q6_K) {
+            if (p.nt == 2) {
+                launch_gemv<WT, 2>(a, grid, s);
+                return hipGetLastError();
+            }
+        }
+        launch_gemv<WT, 1>(a, grid, s);
+    } else switch (p.nt) {
+        case 1:
+            if constexpr (WT == SINTER_Q4_K) launch_gemm<WT, 1>(a, grid, s);
+            break;
+        case 2: launch_gemm<WT, 2>(a, grid, s); break;
+        case 3: launch_gemm<WT, 3>(a, grid, s); break;
+        case 4: launch_gemm<WT, 4>(a, grid, s); break;
+        case 6: launch_gemm<WT, 6>(a, grid, s); break;
+        default: launch_gemm<WT, 8>(a, grid, s); break;
+    }
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_gemv_ubatch(int type, const UbMat *m, uint32_t n, uint32_t nb, const void *xq, uint32_t n_tok,
+                              bool accumulate, hipStream_t s) {
+    UbArgs a = {};
+    a.xq = (const uint8_t *)xq;
+    a.nb = nb;
+    a.n_tok = n_tok;
+    a.accumulate = accumulate;
+    a.n_seg = n;
+    for (uint32_t i = 0; i < n; i++) {
+        a.rows[i] = m[i].rows;
+        a.w[i] = (const uint8_t *)m[i].w;
+        a.y[i] = m[i].y;
+    }
+    return type == SINTER_Q4_K ? launch_ubatch<SINTER_Q4_K>(a, s) : launch_ubatch<SINTER_Q6_K>(a, s);
+}
+
+}  // namespace sinter
+
 extern "C" int sinter_op_gemv_ubatch(int type, const void *w, int64_t rows, int64_t k, const void *xq,
                                      uint32_t n_tokens, float *y, int accumulate, void *stream) {
     if (type != SINTER_Q4_K && type != SINTER_Q6_K)
@@ -547,27 +844,11 @@ extern "C" int sinter_op_gemv_ubatch(int type, const void *w, int64_t rows, int6
     if ((uintptr_t)w % wa || (uintptr_t)xq % 4u || (uintptr_t)y % 4u)
         return set_error(SINTER_ERR_ARG, "gemv_ubatch: alignment (weights %u B, activations and output 4 B)",
                          (unsigned)wa);
-    const uint64_t n_rt = ((uint64_t)rows + UB_WG_ROWS - 1) / UB_WG_ROWS;
-    // token tiles per workgroup: 4 (weights read once per 64 tokens) unless
-    // that leaves fewer than UB_MIN_WGS workgroups; then fewer, the row
-    // tile's token groups running side by side so its weights come from the
-    // memory-side cache after the first
-    uint32_t tpw = UB_TILES;
-    while (tpw > 1 && n_rt * (((uint64_t)n_tokens + UB_TOK * tpw - 1) / (UB_TOK * tpw)) < UB_MIN_WGS) tpw /= 2;
-    const uint64_t n_tg = ((uint64_t)n_tokens + UB_TOK * tpw - 1) / (UB_TOK * tpw);
-    if (n_rt * n_tg > (uint64_t)INT32_MAX) return set_error(SINTER_ERR_ARG, "gemv_ubatch: grid too large");
-    const uint32_t nb = (uint32_t)(k / 256);
-    const dim3 grid((uint32_t)(n_rt * n_tg)), block(UB_THREADS);
-    hipStream_t s = (hipStream_t)stream;
-    if (type == SINTER_Q4_K)
-        hipLaunchKernelGGL(ubatch_gemv_kernel<SINTER_Q4_K>, grid, block, 0, s, (const uint8_t *)w, (uint32_t)rows, nb,
-                           (const uint8_t *)xq, n_tokens, y, (uint32_t)n_tg, tpw,
-                           (uint32_t)(accumulate != 0));
-    else
-        hipLaunchKernelGGL(ubatch_gemv_kernel<SINTER_Q6_K>, grid, block, 0, s, (const uint8_t *)w, (uint32_t)rows, nb,
-                           (const uint8_t *)xq, n_tokens, y, (uint32_t)n_tg, tpw,
-                           (uint32_t)(accumulate != 0));
-    return hip_ok(hipGetLastError(), "gemv_ubatch: launch") ? SINTER_OK : SINTER_ERR_HIP;
+    const UbMat m = {w, y, (uint32_t)rows};
+    const hipError_t e = launch_gemv_ubatch(type, &m, 1, (uint32_t)(k / 256), xq, n_tokens, accumulate != 0,
+                                            (hipStream_t)stream);
+    if (e == hipErrorInvalidValue) return set_error(SINTER_ERR_ARG, "gemv_ubatch: grid too large");
+    return hip_ok(e, "gemv_ubatch: launch") ? SINTER_OK : SINTER_ERR_HIP;
 }
 
 extern "C" int sinter_quant_q8k_ubatch(const float *x, int64_t k, uint32_t n_tokens, void *xq, void *stream) {

@@ -83,6 +83,26 @@ def test_gemv_ubatch_multi_tile_workgroups(sn, orc, torch_gpu, t, rows, k, n_tok
         assert np.array_equal(got[j], orc.gemv(t, w, rows, k, x)), j
 
 
+@pytest.mark.parametrize("t,rows,k,n_tok", [
+    # one case for each compiled split of the launch (token tiles of 16 per
+    # workgroup; few- or many-token kernel), ragged rows and token tails, odd
+    # and even item counts
+    (Q4_K, 41, 1280, 1), (Q4_K, 17, 256, 19),                       # few-token, 1 tile (items % waves != 0)
+    (Q4_K, 8100, 768, 17), (Q4_K, 12289, 512, 20),                  # many-token, 1 and 2 tiles
+    (Q4_K, 12289, 768, 33), (Q4_K, 12289, 512, 63),                 # 3 and 4
+    (Q4_K, 4100, 768, 250), (Q4_K, 8100, 256, 201),                 # 6 and 8
+    (Q6_K, 41, 1280, 1), (Q6_K, 1000, 768, 129),                    # few-token, 1 and 2
+    (Q6_K, 12289, 768, 17), (Q6_K, 12289, 512, 33),                 # many-token, 2 and 3
+    (Q6_K, 3001, 768, 250), (Q6_K, 12289, 512, 65), (Q6_K, 8100, 768, 201)])   # 4, 6 and 8
+def test_gemv_ubatch_every_split(sn, orc, torch_gpu, t, rows, k, n_tok):
+    """Exact sums and the declared fold order: bit-identical on every split."""
+    w = synth_w(sn, t, rows, k, 900 + t + k + rows)
+    xs = activations(k, n_tok, 4000 + rows)
+    got = run_ubatch(sn, orc, torch_gpu, t, w, rows, k, xs)
+    for j, x in enumerate(xs):
+        assert np.array_equal(got[j], orc.gemv(t, w, rows, k, x)), j
+
+
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
 def test_gemv_ubatch_random_block_bytes(sn, orc, torch_gpu, t):
     rows, k, n_tok = 80, 2304, 23           # 9 blocks per row
