@@ -52,7 +52,7 @@ struct GdnUb {
     float *gate, *bgate;  // [T][HV] decay g and beta
     float *state;         // [HV][D][D] (column-major per head), updated in place
     float *o;             // [T][HV*D]
-    uint32_t hk, hv, d, cols, n_tok, c_stride;
+    uint32_t hk, hv, d, n_tok, c_stride;
     float eps, scale;
 };
 
@@ -85,135 +85,152 @@ __global__ __launch_bounds__(256) void gdn_prep_ubatch_kernel(GdnUb a) {
     }
 }
 
-// The delta rule over the ubatch: one (v-head, slice of `cols` state
-// columns) item per workgroup, the decode op_gdn_step's item (gdn.h) with its
-// thread layout and folds -- kv and o as sequential fp32 sums over the
-// thread's RPT rows then lanes_sum_f32 over the column's threads, delta and
-// the update in the same fp32 expressions.  The state slice stays in registers from the first
-// token to the last.  The per-token inputs (precomputed by
-// gdn_prep_ubatch_kernel) move through LDS in stages of GDN_STAGE tokens,
-// double-buffered: stage s + 1 is loaded into registers while stage s is
-// computed, so a token waits on no memory and the workgroup meets at one
-// barrier per stage.
-constexpr uint32_t GDN_STAGE = 16;
-template <uint32_t RPT>
-__global__ __launch_bounds__(256) void gdn_scan_ubatch_kernel(GdnUb a) {
-    // per buffer: k | q [GDN_STAGE][2][D], v [GDN_STAGE][cols], g [GDN_STAGE], beta [GDN_STAGE]
-    constexpr uint32_t BUF = GDN_STAGE * (2 * 256 + 32 + 2);
-    __shared__ __attribute__((aligned(16))) float lds[2 * BUF];
-    const uint32_t D = a.d, HK = a.hk, HV = a.hv, cols = a.cols, tpc = 256u / cols;
-    const uint32_t slices = D / cols, item = blockIdx.x, tid = threadIdx.x;
-    const uint32_t h = item / slices, c0 = (item % slices) * cols, hk = h % HK;
-    const uint32_t col = c0 + tid / tpc, i0 = (tid % tpc) * RPT;
-    const uint32_t kq_f = GDN_STAGE * 2 * D, v_off = kq_f, g_off = v_off + GDN_STAGE * cols, b_off = g_off + GDN_STAGE;
-    float *srow = a.state + ((size_t)h * D + col) * D + i0;
+// The delta rule over the ubatch: one wave per (v-head, 64 / TPC state
+// columns), the decode op_gdn_step's column layout and folds (gdn.h): TPC
+// threads of RPT rows per column, kv and o as sequential fp32 sums over the
+// thread's rows then lanes_sum_f32 over the column's threads, delta and the
+// update in the same fp32 expressions.  The state stays in registers from the
+// first token to the last.
+//
+// A token is a dependent chain (kv sum -> delta -> update -> sums) of 7 RPT
+// instructions, one wave's own issue rate: what else a token waits for decides
+// the time.  k and q come by LDS-DMA, GDN_STAGE tokens at a time and one stage
+// ahead, in the order the lanes read them -- position j TPC + p holds rows
+// RPT p + 4j .. + 3, so the TPC threads of a column read consecutive 16-byte
+// units (row order put them 64 bytes apart, four to a bank) -- and are read
+// into registers a token ahead; a stage belongs to one wave, so there is no
+// barrier.  27B shapes, 256 tokens: 139 us with four-wave workgroups, row
+// order and a barrier per stage, 80 us so.
+constexpr uint32_t GDN_STAGE = 8;
+static_assert(GDN_STAGE <= 8, "a stage's outputs fit the threads of a column");
+template <uint32_t RPT, uint32_t TPC>
+__global__ __launch_bounds__(64) void gdn_scan_ubatch_kernel(GdnUb a) {
+    constexpr uint32_t D = RPT * TPC, COLS = 64u / TPC, VEC = D * 4u, BUF = GDN_STAGE * 2u * VEC;
+    __shared__ __attribute__((aligned(16))) unsigned char sm[2 * BUF];
+    LDS unsigned char *L = (LDS unsigned char *)sm;
+    const uint32_t lbase = (uint32_t)(uintptr_t)L;
+    const uint32_t HK = a.hk, HV = a.hv, lane = threadIdx.x, p = lane % TPC;
+    const uint32_t h = blockIdx.x / (D / COLS), col = (blockIdx.x % (D / COLS)) * COLS + lane / TPC, hk = h % HK;
+    const uint32_t n = a.n_tok, last = n - 1u;
+    float *srow = a.state + ((size_t)h * D + col) * D + p * RPT;
     float s[RPT];
+    auto load = [&](const LDS unsigned char *v, float (&d)[RPT]) {
+#pragma unroll
+        for (uint32_t j = 0; j < RPT / 4; j++) {
+            const f32x4 t = *reinterpret_cast<const LDS f32x4 *>(v + 16u * (j * TPC + p));
+            d[4 * j] = t.x; d[4 * j + 1] = t.y; d[4 * j + 2] = t.z; d[4 * j + 3] = t.w;
+        }
+    };
 #pragma unroll
     for (uint32_t r = 0; r < RPT; r += 4) {
         const f32x4 t = *reinterpret_cast<const f32x4 *>(srow + r);
         s[r] = t.x; s[r + 1] = t.y; s[r + 2] = t.z; s[r + 3] = t.w;
     }
-    // stage loads into registers: thread tid takes float4 j = tid + 256 i of
-    // the k|q block (token j / (D / 2), half (j / (D / 4)) % 2, element
-    // 4 (j % (D / 4))); threads below GDN_STAGE cols / 4 one float4 of v;
-    // threads 128 .. 128 + 2 GDN_STAGE one g or beta
-    constexpr uint32_t KQ4 = GDN_STAGE * 2 * 256 / 4 / 256;   // float4 per thread at D = 256
-    const uint32_t n_kq4 = kq_f / 4, n_v4 = GDN_STAGE * cols / 4;
-    f32x4 rkq[KQ4];
-    f32x4 rv = {0.0f, 0.0f, 0.0f, 0.0f};
-    float rg = 0.0f;
-    const uint32_t nst = (a.n_tok + GDN_STAGE - 1) / GDN_STAGE;
-    auto issue = [&](uint32_t st) {
+    // stage st's inputs: k | q of its tokens into buffer st & 1, v of the
+    // lane's column, g and beta of token lane % GDN_STAGE in registers
+    // (tokens past the last repeat it, never used)
+    struct Small { float v[GDN_STAGE], g, b; };
+    auto issue = [&](uint32_t st, Small &w) {
         const uint32_t tb = st * GDN_STAGE;
 #pragma unroll
-        for (uint32_t i = 0; i < KQ4; i++) {
-            const uint32_t j = tid + 256u * i;
-            if (j < n_kq4) {
-                const uint32_t tk = j / (D / 2), half = (j / (D / 4)) & 1u, e = 4u * (j % (D / 4));
-                const uint32_t t = min(tb + tk, a.n_tok - 1);
-                const float *src = (half ? a.qn : a.kn) + ((size_t)t * HK + hk) * D + e;
-                rkq[i] = *reinterpret_cast<const f32x4 *>(src);
-            }
+        for (uint32_t i = 0; i < BUF / 1024u; i++) {
+            const uint32_t u = 64u * i + lane, tk = u / (D / 2), half = (u / (D / 4)) & 1u, pos = u % (D / 4);
+            const uint32_t t = min(tb + tk, last), c = (pos % TPC) * (RPT / 4) + pos / TPC;
+            // (byte offset from the first token: kn follows qn in one buffer)
+            const uint32_t voff = (((half ? 0u : n) + t) * HK + hk) * VEC + 16u * c;
+            lds_dma16<false>((uintptr_t)a.qn, voff, lbase + (st & 1u) * BUF + 1024u * i);
         }
-        if (tid < n_v4) {
-            const uint32_t tk = tid / (cols / 4), e = 4u * (tid % (cols / 4));
-            const uint32_t t = min(tb + tk, a.n_tok - 1);
-            rv = *reinterpret_cast<const f32x4 *>(a.qkv + (size_t)t * a.c_stride + (size_t)2 * HK * D +
-                                                  (size_t)h * D + c0 + e);
-        }
-        if (tid >= 128 && tid < 128 + 2 * GDN_STAGE) {
-            const uint32_t tk = (tid - 128) % GDN_STAGE, t = min(tb + tk, a.n_tok - 1);
-            rg = tid < 128 + GDN_STAGE ? a.gate[(size_t)t * HV + h] : a.bgate[(size_t)t * HV + h];
-        }
-    };
-    auto park = [&](uint32_t st) {
-        float *L = lds + (st & 1u) * BUF;
+        const uint32_t tg = min(tb + lane % GDN_STAGE, last);
+        w.g = a.gate[(size_t)tg * HV + h];
+        w.b = a.bgate[(size_t)tg * HV + h];
 #pragma unroll
-        for (uint32_t i = 0; i < KQ4; i++) {
-            const uint32_t j = tid + 256u * i;
-            if (j < n_kq4) *reinterpret_cast<f32x4 *>(L + 4 * j) = rkq[i];
-        }
-        if (tid < n_v4) *reinterpret_cast<f32x4 *>(L + v_off + 4 * tid) = rv;
-        if (tid >= 128 && tid < 128 + 2 * GDN_STAGE) L[g_off + (tid - 128)] = rg;
+        for (uint32_t i = 0; i < GDN_STAGE; i++)
+            w.v[i] = a.qkv[(size_t)min(tb + i, last) * a.c_stride + (size_t)2 * HK * D + (size_t)h * D + col];
     };
-    issue(0);
-    park(0);
-    if (nst > 1) issue(1);
-    __syncthreads();
-    // Token t's o sum and token t + 1's kv sum take the same updated state
-    // and run in one loop, two independent chains; the kv sum of a stage's
-    // first token runs alone after the stage barrier.
-    auto load8 = [&](const float *p, float (&d)[RPT]) {
+    // the stage has landed: its last load has, and loads complete in order
+    auto landed = [&](Small &w) { asm volatile("" : "+v"(w.v[GDN_STAGE - 1])::"memory"); };
+    auto kvec = [&](uint32_t st, uint32_t i) { return L + (st & 1u) * BUF + i * 2u * VEC; };
+    auto qvec = [&](uint32_t st, uint32_t i) { return L + (st & 1u) * BUF + i * 2u * VEC + VEC; };
+    const uint32_t nst = (n + GDN_STAGE - 1) / GDN_STAGE;
+    Small cur, nxt;
+    issue(0, cur);
+    landed(cur);
+    float kc[RPT], qc[RPT], kn[RPT];
+    load(kvec(0, 0), kc);
+    load(qvec(0, 0), qc);
+    float dkv = 0.0f;
 #pragma unroll
-        for (uint32_t r = 0; r < RPT; r += 4) {
-            const f32x4 v = *reinterpret_cast<const f32x4 *>(p + r);
-            d[r] = v.x; d[r + 1] = v.y; d[r + 2] = v.z; d[r + 3] = v.w;
-        }
-    };
-    for (uint32_t st = 0; st < nst; st++) {
-        const float *L = lds + (st & 1u) * BUF;
-        const uint32_t tb = st * GDN_STAGE, te = min(GDN_STAGE, a.n_tok - tb);
-        float kk[RPT], qq[RPT], kn[RPT];
-        load8(L + i0, kk);
-        float dkv = 0.0f;
+    for (uint32_t r = 0; r < RPT; r++) {
+        const float pr = s[r] * kc[r];
+        dkv = dkv + pr;
+    }
+    dkv = lanes_sum_f32(dkv, TPC);
+    load(kvec(0, 1), kn);
+    // one token: its update and o sum beside the next token's kv sum (two
+    // independent chains on the same updated state)
+    auto token = [&](float vcol, float g, float beta) -> float {
+        float u1[RPT];
+#pragma unroll
+        for (uint32_t r = 0; r < RPT; r++) u1[r] = g * s[r];
+        const float t1 = g * dkv;
+        const float t2 = vcol - t1;
+        const float delta = t2 * beta;
+        float dout = 0.0f, dkn = 0.0f;
 #pragma unroll
         for (uint32_t r = 0; r < RPT; r++) {
-            const float pr = s[r] * kk[r];
-            dkv = dkv + pr;
+            const float u2 = kc[r] * delta;
+            s[r] = u1[r] + u2;
+            const float po = s[r] * qc[r], pn = s[r] * kn[r];
+            dout = dout + po;
+            dkn = dkn + pn;
         }
-        dkv = lanes_sum_f32(dkv, tpc);
-        for (uint32_t tk = 0; tk < te; tk++) {
-            const uint32_t tn = tk + 1 < te ? tk + 1 : tk;   // (the last token's "next" sum is dropped)
-            load8(L + tk * 2 * D + D + i0, qq);
-            load8(L + tn * 2 * D + i0, kn);
-            const float vcol = L[v_off + tk * cols + (col - c0)];
-            const float g = L[g_off + tk], beta = L[b_off + tk];
-            const float kvf = dkv;
-            const float t1 = g * kvf;
-            const float t2 = vcol - t1;
-            const float delta = t2 * beta;
-            float dout = 0.0f, dkn = 0.0f;
+        dkv = lanes_sum_f32(dkn, TPC);
+        return lanes_sum_f32(dout, TPC) * a.scale;
+    };
+    float *orow = a.o + (size_t)h * D + col;
+    auto lane_f = [](float v, uint32_t i) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), (int)i));
+    };
+    uint32_t st = 0;
+    // whole stages (kc, qc of the stage's first token and kn of the one after
+    // it are loaded, dkv is the first token's)
+    for (; (st + 1) * GDN_STAGE <= n; st++) {
+        // its buffer was last read in the stage before; the reads still in
+        // flight are at most the last token's prefetch, from the other buffer
+        // (LDS reads complete in order)
+        asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(RPT / 2 < 15 ? RPT / 2 : 15) : "memory");
+        issue(min(st + 1, nst - 1), nxt);
+        const uint32_t tb = st * GDN_STAGE;
+        float ov = 0.0f;   // token tb + p's output (every thread of a column has it: one store per stage)
 #pragma unroll
-            for (uint32_t r = 0; r < RPT; r++) {
-                const float u1 = g * s[r];
-                const float u2 = kk[r] * delta;
-                s[r] = u1 + u2;
-                const float po = s[r] * qq[r], pn = s[r] * kn[r];
-                dout = dout + po;
-                dkn = dkn + pn;
-            }
-            dout = lanes_sum_f32(dout, tpc);
-            dkv = lanes_sum_f32(dkn, tpc);
-            if ((tid % tpc) == 0) a.o[(size_t)(tb + tk) * HV * D + (size_t)h * D + col] = dout * a.scale;
+        for (uint32_t i = 0; i < GDN_STAGE; i++) {
+            float qx[RPT], kx[RPT];   // the next token's q, the k after that
+            if (i == GDN_STAGE - 2) landed(nxt);
+            load(i + 1 < GDN_STAGE ? qvec(st, i + 1) : qvec(st + 1, 0), qx);
+            load(i + 2 < GDN_STAGE ? kvec(st, i + 2) : kvec(st + 1, i + 2 - GDN_STAGE), kx);
+            const float o = token(cur.v[i], lane_f(cur.g, i), lane_f(cur.b, i));
+            ov = p == i ? o : ov;
 #pragma unroll
-            for (uint32_t r = 0; r < RPT; r++) kk[r] = kn[r];
+            for (uint32_t r = 0; r < RPT; r++) { kc[r] = kn[r]; qc[r] = qx[r]; kn[r] = kx[r]; }
         }
-        if (st + 1 < nst) {
-            park(st + 1);   // (its buffer was last read in stage st - 1, before the last barrier)
-            if (st + 2 < nst) issue(st + 2);
-        }
-        __syncthreads();
+        if (TPC == GDN_STAGE || p < GDN_STAGE) orow[(size_t)(tb + p) * HV * D] = ov;
+        cur = nxt;
     }
+    // the last, partial stage (already staged; sums for tokens past the end are dropped)
+    for (uint32_t i = 0; i < n - st * GDN_STAGE; i++) {
+        const uint32_t i1 = min(i + 1, GDN_STAGE - 1), i2 = min(i + 2, GDN_STAGE - 1);
+        float qx[RPT], kx[RPT];
+        load(qvec(st, i1), qx);
+        load(kvec(st, i2), kx);
+        float v = cur.v[0];
+#pragma unroll
+        for (uint32_t j = 1; j < GDN_STAGE; j++) v = i == j ? cur.v[j] : v;
+        const float o = token(v, lane_f(cur.g, i), lane_f(cur.b, i));
+        if (p == 0) orow[(size_t)(st * GDN_STAGE + i) * HV * D] = o;
+#pragma unroll
+        for (uint32_t r = 0; r < RPT; r++) { kc[r] = kn[r]; qc[r] = qx[r]; kn[r] = kx[r]; }
+    }
+    dma_wait();   // (the last staging must not outlive the wave's LDS)
 #pragma unroll
     for (uint32_t r = 0; r < RPT; r += 4) {
         const f32x4 v = {s[r], s[r + 1], s[r + 2], s[r + 3]};
@@ -641,17 +658,16 @@ hipError_t launch_gdn_ubatch(const float *qkv, const float *alpha, const float *
     a.kn = a.qn + (size_t)n_tok * hk * d;
     a.gate = a.kn + (size_t)n_tok * hk * d;
     a.bgate = a.gate + (size_t)n_tok * hv;
-    a.hk = hk; a.hv = hv; a.d = d; a.cols = d >= 128 ? 32u : 16u; a.n_tok = n_tok;
+    a.hk = hk; a.hv = hv; a.d = d; a.n_tok = n_tok;
     a.c_stride = (2 * hk + hv) * d;
     a.eps = eps; a.scale = scale;
-    const uint32_t items = hv * (d / a.cols), rpt = d / (256u / a.cols);
     if (n_tok == 0) return hipSuccess;
     hipLaunchKernelGGL(gdn_prep_ubatch_kernel, dim3(n_tok, hk), dim3(256), 0, s, a);
-    switch (rpt) {
-    case 4: hipLaunchKernelGGL(gdn_scan_ubatch_kernel<4>, dim3(items), dim3(256), 0, s, a); break;
-    case 8: hipLaunchKernelGGL(gdn_scan_ubatch_kernel<8>, dim3(items), dim3(256), 0, s, a); break;
-    case 16: hipLaunchKernelGGL(gdn_scan_ubatch_kernel<16>, dim3(items), dim3(256), 0, s, a); break;
-    case 32: hipLaunchKernelGGL(gdn_scan_ubatch_kernel<32>, dim3(items), dim3(256), 0, s, a); break;
+    // the decode op's threads per column: 256 / cols, cols 32 (16 at d = 64)
+    switch (d) {
+    case 64: hipLaunchKernelGGL((gdn_scan_ubatch_kernel<4, 16>), dim3(hv * 16), dim3(64), 0, s, a); break;
+    case 128: hipLaunchKernelGGL((gdn_scan_ubatch_kernel<16, 8>), dim3(hv * 16), dim3(64), 0, s, a); break;
+    case 256: hipLaunchKernelGGL((gdn_scan_ubatch_kernel<32, 8>), dim3(hv * 32), dim3(64), 0, s, a); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

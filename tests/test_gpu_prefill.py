@@ -185,3 +185,26 @@ def test_batched_prefill_gdn_head_sizes(sn, torch_gpu, d, hk, hv):
     finally:
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("d,hk,hv", [(64, 2, 4), (128, 2, 4), (256, 1, 2)])
+def test_batched_prefill_gdn_stage_edges(sn, torch_gpu, d, hk, hv):
+    """The GDN scan takes 8 tokens per stage: ubatches of 1, 7, 8, 9, 15, 16
+    and 17 tokens (whole and partial last stages) against one pass per token."""
+    cfg = small_config(sn, n_layer=2, n_ctx=128)
+    cfg.gdn_d, cfg.gdn_hk, cfg.gdn_hv = d, hk, hv
+    toks = [int(t) for t in np.random.default_rng(d + 1).integers(0, cfg.n_vocab, 73)]
+    a, b = sn.Model(cfg, seed=53), sn.Model(cfg, seed=53)
+    try:
+        pos = 0
+        for n in (1, 7, 8, 9, 15, 16, 17):
+            print(f"gdn stages d={d}: {n} tokens at {pos}", flush=True)
+            nxt_a = a.prefill(toks[pos:pos + n], pos, mode="batched")
+            nxt_b = b.prefill(toks[pos:pos + n], pos, mode="tokenwise")
+            pos += n
+            assert nxt_a == nxt_b
+            assert np.array_equal(a.logits(), b.logits())
+            same_state(a, b, cfg)
+    finally:
+        a.close()
+        b.close()
