@@ -18,6 +18,8 @@
 // prefill query is the decode's declared fp32 fold over one chunk holding all
 // its positions (the decode splits long contexts over chunks); the oracle's
 // or_attn_prefill restates it.
+#include <algorithm>
+
 #include "internal.h"
 #include "gemv.h"
 #include "attn.h"
@@ -699,8 +701,12 @@ hipError_t launch_attn_prefill(const float *qr, const float *qg, const void *kc,
     a.nq = nq; a.nkv = nkv; a.hd = hd; a.kv_type = kv_type; a.n_chunks = n_chunks; a.chunk_min = chunk_min;
     a.scale = scale;
     if (n_tok == 0) return hipSuccess;
-    // chunks of the deepest query (the others have as many or fewer)
-    const uint32_t cmax = att_geom((uint32_t)pos0 + n_tok, n_chunks, chunk_min).n;
+    // the most chunks any of the queries is split into: not the deepest one's,
+    // whose tiles per chunk may just have grown (64 chunks of 4 tiles up to
+    // 8192 positions, 52 of 5 at 8193)
+    uint32_t cmax = 0;
+    for (uint32_t n_kv = (uint32_t)pos0 + 1; n_kv <= (uint32_t)pos0 + n_tok; n_kv = (n_kv + 31u) / 32u * 32u + 1u)
+        cmax = std::max(cmax, att_geom(n_kv, n_chunks, chunk_min).n);
     const uint32_t items = nkv * cmax * (nq / nkv) * ((n_tok + PF_SLOTS - 1) / PF_SLOTS);
     if (kv_type == SINTER_Q8_0)
         hipLaunchKernelGGL(attn_prefill_split_kernel<true>, dim3(items), dim3(256), 0, s, a, cmax);

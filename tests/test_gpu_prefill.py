@@ -208,3 +208,24 @@ def test_batched_prefill_gdn_stage_edges(sn, torch_gpu, d, hk, hv):
     finally:
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("past,n,chunks,cmin", [(78, 33, 3, 32), (8180, 40, 64, 128)])
+def test_batched_prefill_across_a_change_of_tiles_per_chunk(sn, torch_gpu, past, n, chunks, cmin):
+    """Where the tiles per chunk grow inside a ubatch, its shallower queries
+    are split into more chunks than its deepest one (8192 positions: 64
+    chunks, 8193: 52): every chunk of every query is computed."""
+    cfg = small_config(sn, n_layer=2, n_ctx=past + n + 8)
+    cfg.attn_every, cfg.attn_chunks, cfg.attn_chunk_min = 1, chunks, cmin
+    toks = [int(t) for t in np.random.default_rng(past).integers(0, cfg.n_vocab, n)]
+    a, b = sn.Model(cfg, seed=61), sn.Model(cfg, seed=61)
+    try:
+        a.synth_context(past, seed=62)
+        b.synth_context(past, seed=62)
+        print(f"prefill of {n} tokens at {past}, {chunks} chunks", flush=True)
+        assert a.prefill(toks, past, mode="batched") == b.prefill(toks, past, mode="tokenwise")
+        assert np.array_equal(a.logits(), b.logits())
+        same_state(a, b, cfg)
+    finally:
+        a.close()
+        b.close()
