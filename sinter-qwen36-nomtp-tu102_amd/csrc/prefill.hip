@@ -10,14 +10,13 @@
 //                            token, the state slice in registers
 //   attn_prep_ubatch_kernel  q/k RMSNorm + NEOX RoPE per token and head, the
 //                            ubatch's K/V rows appended to the cache
-//   attn_prefill_kernel      causal attention of the ubatch's queries over
-//                            the cache, gated by sigmoid(gate)
-// The first three compute what the decode ops compute, expression for
-// expression (same helpers, same fp64 folds), so a prefilled state and KV
-// cache are bit-identical to the decode program's.  The attention of a
-// prefill query is the decode's declared fp32 fold over one chunk holding all
-// its positions (the decode splits long contexts over chunks); the oracle's
-// or_attn_prefill restates it.
+//   attn_prefill_split_kernel, attn_prefill_merge_kernel
+//                            causal attention of the ubatch's queries over
+//                            the cache, split over chunks and merged as the
+//                            decode does, gated by sigmoid(gate)
+// All compute what the decode ops compute, expression for expression (same
+// helpers, same fp64 folds, same chunks), so a prefilled state, KV cache and
+// logits are bit-identical to the decode program's.
 #include <algorithm>
 
 #include "internal.h"
@@ -355,37 +354,56 @@ struct AttnPrefill {
     float scale;
 };
 
-constexpr uint32_t PF_SLOTS = 8;   // queries per work item
-// K/V tile buffers of the prefill attention: with PF_NBUF = 2 (tile j + 1
-// loads while tile j is computed) the workgroup's LDS fits two workgroups
-// per CU; 3 keeps two tiles in flight as the decode does.
-#ifndef PF_NBUF
-#define PF_NBUF 2
-#endif
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+constexpr uint32_t PF_SLOTS = 16;   // queries per work item: the MFMA's 16
+// K/V tile buffers (tile j + 1 loads while tile j is computed): two, so that
+// the workgroup's LDS fits two workgroups per CU
+constexpr uint32_t PF_NBUF = 2;
 constexpr uint32_t PF_Q8_KC = 2 * PF_NBUF * ATT_Q8_RAWB, PF_Q8_VC = PF_Q8_KC + 32 * 256;
 constexpr uint32_t PF_Q8_KS = PF_Q8_VC + 32 * 256, PF_Q8_VS = PF_Q8_KS + 32 * 8 * 4;
-constexpr uint32_t PF_TILES = PF_NBUF * ATT_F16_BUF > 8u * PF_SLOTS * 256u * 4u ? PF_NBUF * ATT_F16_BUF
-                                                                               : 8u * PF_SLOTS * 256u * 4u;
+constexpr uint32_t PF_COMB = 8u * 8u * 256u * 4u;   // the row groups' V sums of 8 queries
+constexpr uint32_t PF_TILES = PF_NBUF * ATT_F16_BUF > PF_COMB ? PF_NBUF * ATT_F16_BUF : PF_COMB;
 static_assert(PF_Q8_VS + 32 * 8 * 4 <= PF_TILES, "Q8_0 tiles fit the tile region");
 
-// Work item = (kv head g, split chunk c, q head hh of g's group, block of 8
+// Work item = (kv head g, split chunk c, q head hh of g's group, block of 16
 // consecutive queries), the block index running over the query blocks
-// first, so the items that read one chunk of one kv head run side by side.  Query i of the ubatch (position pos0 + i) is split
-// exactly as the decode splits it at that position: att_geom(pos0 + i + 1,
+// first, so the items that read one chunk of one kv head run side by side.
+// Query i of the ubatch (position pos0 + i) is split exactly as the decode splits it at that position: att_geom(pos0 + i + 1,
 // C, chunk_min) chunks of tpc tiles, chunk c holding rows [c tpc 32,
-// min((c + 1) tpc 32, pos0 + i + 1)).  The item runs the decode attention's
-// tile loop (attn.h) over the union of its queries' chunk-c rows with the
-// register slots holding 8 queries of one head instead of the 8 heads of one
-// query, so every K/V tile is read once for 8 queries; a row outside a
+// min((c + 1) tpc 32, pos0 + i + 1)).  The item runs the union of its
+// queries' chunk-c rows in the decode attention's tiles; a row outside a
 // query's own range is masked out of its scores and enters its V sums as
 // fmaf(0, v, acc) (no change but the sign of a zero sum, which the Q8_K
 // quantisation of the attention output erases).  Per query the chunk partial
 // -- the 8 row groups merged, O, M, L -- is the decode's, bit for bit.
+//
+// The decode's fmaf chains run on v_mfma_f32_16x16x1_4b_f32: four 16 x 16
+// blocks, one product each, every output a single fmaf (checked bit for bit,
+// subnormals included), at twice the VALU's rate and without the lanes'
+// exchanges:
+//   scores  wave w takes the dims of the decode's lanes p in {w, 15 - w,
+//           7 - w, 8 + w} (a block each) and p + 16: blocks of 16 rows (A) x
+//           16 queries (B) over the 8 dims of each p, ascending.  The first
+//           three levels of the decode's sum over the lanes (masks 16, 15, 7)
+//           are then adds between registers of a lane, the last two (2, 1)
+//           adds of the four waves' results, exchanged through LDS.
+//   V sums  wave w holds row groups 2w and 2w + 1: 16 queries (A, their
+//           weights of one row) x 64 dims (B) per MFMA, lane l's B being dim
+//           4l + jj of the row; the groups' 4 rows of a tile ascending.
+// The softmax state of row groups 2w and 2w + 1 lives in wave w (a thread per
+// two rows and query), so only the scores cross waves: one barrier beside the
+// tile's.  K rows lie in LDS as 16-byte chunks, chunk p at slot p ^ (row %
+// 16), so 16 rows' reads of one chunk hit distinct banks.  256 queries behind
+// 8192 positions, 27B shapes: 1.60 ms with VALU chains (8 queries per item),
+// 0.98 ms so.
 template <bool Q8>
-__global__ __launch_bounds__(256) void attn_prefill_split_kernel(AttnPrefill a, uint32_t cmax) {
+__global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(AttnPrefill a, uint32_t cmax) {
     __shared__ __attribute__((aligned(16))) unsigned char tiles[PF_TILES];
-    __shared__ __attribute__((aligned(16))) float wl[8 * (4 * PF_SLOTS + PF_SLOTS)];
-    __shared__ __attribute__((aligned(16))) float gm[2 * 8 * PF_SLOTS];
+    __shared__ __attribute__((aligned(16))) float sx[4 * 32 * PF_SLOTS];         // scores: [wave][row][query]
+    __shared__ __attribute__((aligned(16))) float wl[32 * PF_SLOTS + 8 * PF_SLOTS];   // weights [row][query], corrections [group][query]
+    __shared__ __attribute__((aligned(16))) float gm[2 * 8 * PF_SLOTS];           // m, l [group][query]
     const uint32_t t = threadIdx.x, HD = a.hd, NQ = a.nq, NKV = a.nkv, gqa = NQ / NKV, C = a.n_chunks;
     const uint32_t n_qb = (a.n_tok + PF_SLOTS - 1) / PF_SLOTS;
     uint32_t it = blockIdx.x;
@@ -393,43 +411,43 @@ __global__ __launch_bounds__(256) void attn_prefill_split_kernel(AttnPrefill a, 
     const uint32_t hh = it % gqa; it /= gqa;
     const uint32_t c = it % cmax, g = it / cmax;
     const uint32_t head = g * gqa + hh, q0 = qb * PF_SLOTS, nqs = min(PF_SLOTS, a.n_tok - q0);
-    // query s's chunk-c rows [k0, k1) (empty when its split has fewer chunks)
-    auto range = [&](uint32_t s, uint32_t &k0, uint32_t &k1) {
-        const uint32_t n_kv = (uint32_t)a.pos0 + q0 + s + 1u;
+    const uint32_t lane = t & 63u, w = __builtin_amdgcn_readfirstlane(t >> 6), l16 = lane & 15u, lb = lane >> 4;
+    // the chunk-c rows [k0, k1) of query `lane % 16` (empty when its split has
+    // fewer chunks), and their union U0, U1 over the item's queries
+    uint32_t k0 = 0, k1 = 0;
+    if (l16 < nqs) {
+        const uint32_t n_kv = (uint32_t)a.pos0 + q0 + l16 + 1u;
         const AttGeom geo = att_geom(n_kv, C, a.chunk_min);
-        k0 = k1 = 0;
-        if (s < nqs && c < geo.n) {
+        if (c < geo.n) {
             k0 = c * geo.tpc * ATT_TILE;
             k1 = min(k0 + geo.tpc * ATT_TILE, n_kv);
         }
-    };
-    uint32_t U0 = 0xffffffffu, U1 = 0;
-    for (uint32_t s = 0; s < nqs; s++) {
-        uint32_t k0, k1;
-        range(s, k0, k1);
-        if (k1 > k0) {
-            U0 = min(U0, k0);
-            U1 = max(U1, k1);
-        }
     }
+    uint32_t U0 = k1 > k0 ? k0 : 0xffffffffu, U1 = k1;
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) {
+        U0 = min(U0, (uint32_t)__shfl_xor((int)U0, o, 64));
+        U1 = max(U1, (uint32_t)__shfl_xor((int)U1, o, 64));
+    }
+    U0 = __builtin_amdgcn_readfirstlane(U0);
+    U1 = __builtin_amdgcn_readfirstlane(U1);
     if (U1 == 0) return;   // (uniform) no query of the block has a chunk c
     const uint32_t ntile = (U1 - U0 + ATT_TILE - 1) / ATT_TILE;
     const uint32_t HB = Q8 ? ATT_Q8_HEAD : HD * 2u, RWB = NKV * HB;
-    const uint32_t w = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63u;
     LDS unsigned char *Lu = (LDS unsigned char *)tiles;
     const uint32_t kbase = (uint32_t)(uintptr_t)Lu;
-    // tile j (rows U0 + 32 j ..) into buffer j % PF_NBUF, as the decode's
-    // issue_tile; rows past U1 re-read row U1 - 1
+    // tile j (rows U0 + 32 j ..) into buffer j % PF_NBUF; rows past U1 re-read
+    // row U1 - 1
     auto issue_tile = [&](uint32_t j) {
         const uint32_t t0 = U0 + j * ATT_TILE;
         if constexpr (!Q8) {
             const uint32_t bo = (j % PF_NBUF) * ATT_F16_BUF;
 #pragma unroll
             for (uint32_t kk = 0; kk < 4; kk++) {
-                const uint32_t k = w + 4 * kk, row = min(t0 + 2 * k + (lane >> 5), U1 - 1);
-                const uint32_t voff = row * RWB + g * HB + (lane & 31) * 16;
-                lds_dma16<false>((uintptr_t)a.kc, voff, kbase + bo + k * 1024);
-                lds_dma16<false>((uintptr_t)a.vc, voff, kbase + bo + ATT_TILE * 512 + k * 1024);
+                const uint32_t k = w + 4 * kk, r = 2 * k + (lane >> 5), row = min(t0 + r, U1 - 1);
+                const uint32_t off = row * RWB + g * HB, slot = lane & 31;
+                lds_dma16<false>((uintptr_t)a.kc, off + (slot ^ (r & 15u)) * 16, kbase + bo + k * 1024);
+                lds_dma16<false>((uintptr_t)a.vc, off + slot * 16, kbase + bo + ATT_TILE * 512 + k * 1024);
             }
         } else {
             const uint32_t rb = (j % PF_NBUF) * 2 * ATT_Q8_RAWB;
@@ -443,47 +461,53 @@ __global__ __launch_bounds__(256) void attn_prefill_split_kernel(AttnPrefill a, 
         }
     };
     issue_tile(0);
-    if (PF_NBUF > 2 && ntile > 1) issue_tile(1);
-    const uint32_t rr = t >> 5, p = t & 31, mp = att_perm(p);
-    // register slot s holds query q0 + (s ^ (mp & 7)) of head `head` (zero past the ubatch)
-    float qv[PF_SLOTS][8], acc[PF_SLOTS][8];
+    // score operands: block lb of the MFMAs holds lane group p = xp (+ 16)
+    const uint32_t xp = lb == 0 ? w : lb == 1 ? 15u - w : lb == 2 ? 7u - w : 8u + w;
+    float qv[2][8];
 #pragma unroll
-    for (uint32_t s = 0; s < PF_SLOTS; s++) {
-        const uint32_t qi = s ^ (mp & 7u);
-        const bool ok = qi < nqs;
-        const float *src = a.qr + ((size_t)(q0 + (ok ? qi : 0u)) * NQ + head) * HD + 8 * p;
+    for (uint32_t j = 0; j < 2; j++) {
+        const bool ok = l16 < nqs;
+        const float *src = a.qr + ((size_t)(q0 + (ok ? l16 : 0u)) * NQ + head) * HD + 8 * (xp + 16 * j);
         const float4 v0 = reinterpret_cast<const float4 *>(src)[0], v1 = reinterpret_cast<const float4 *>(src)[1];
         const float q8v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
 #pragma unroll
-        for (uint32_t d = 0; d < 8; d++) {
-            qv[s][d] = ok ? q8v[d] : 0.0f;
-            acc[s][d] = 0.0f;
-        }
+        for (uint32_t d = 0; d < 8; d++) qv[j][d] = ok ? q8v[d] : 0.0f;
+        // (waited for here: the loop's waits would be for the next tile's DMA too)
+#pragma unroll
+        for (uint32_t d = 0; d < 8; d++) asm volatile("" : "+v"(qv[j][d]));
     }
-    // softmax state of (row group rr, query my_s): the same in the group's 4 lanes of that query
+    const f32x16 z16 = {0.0f};
+    f32x16 acc[2][4];   // V sums: [row group 2w + gi][jj]: query 4 lb + v, dim 64 b + 4 l16 + jj at element 4 b + v
+#pragma unroll
+    for (uint32_t gi = 0; gi < 2; gi++)
+#pragma unroll
+        for (uint32_t jj = 0; jj < 4; jj++) acc[gi][jj] = z16;
+    // softmax: this thread's row group, query, and pair of the group's rows of a tile
+    const uint32_t rr = t >> 5, sq = (t >> 1) & 15u, hf = t & 1u;
+    const uint32_t my0 = (uint32_t)__shfl((int)k0, (int)sq, 64), my1 = (uint32_t)__shfl((int)k1, (int)sq, 64);
     float mrun = -INFINITY, lrun = 0.0f;
-    const uint32_t my_s = mp & 7u, my_i = mp >> 3;
-    uint32_t my0, my1;
-    range(my_s, my0, my1);
-    LDS float *wgr = (LDS float *)wl + rr * (4 * PF_SLOTS + PF_SLOTS);
-    LDS float *gml = (LDS float *)gm;
+    LDS float *S = (LDS float *)sx, *W = (LDS float *)wl, *CF = W + 32 * PF_SLOTS, *gml = (LDS float *)gm;
 
     for (uint32_t j = 0; j < ntile; j++) {
         const uint32_t t0 = U0 + j * ATT_TILE, b = j % PF_NBUF;
-        if (PF_NBUF > 2 && j + 1 < ntile) {
-            // tile j landed; tile j+1 may still fly
-            if (Q8) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-        } else {
-            dma_wait();
-        }
+        dma_wait();
         __syncthreads();   // tile j landed for every wave; every wave is past tile j - 1
-        if (j + PF_NBUF - 1 < ntile) issue_tile(j + PF_NBUF - 1);   // into the buffer tile j - 1 used
+        if (j + 1 < ntile) issue_tile(j + 1);   // into the buffer tile j - 1 used
         const LDS unsigned char *kt = Lu + b * ATT_F16_BUF, *vt = kt + ATT_TILE * 512;
         if constexpr (Q8) {
+            // thread t: block bb of row rq; K codes as 16-byte chunks, chunk i
+            // at slot i ^ (row % 16)
             const uint32_t rq = t >> 3, bb = t & 7u, rb = b * 2 * ATT_Q8_RAWB;
             const LDS unsigned char *raw = Lu + rb + rq * ATT_Q8_HEAD + 34u * bb;
-            att_q8_split(raw, Lu + PF_Q8_KC + rq * 256 + 32u * bb, reinterpret_cast<LDS float *>(Lu + PF_Q8_KS) + t);
+            const LDS uint16_t *hw = reinterpret_cast<const LDS uint16_t *>(raw);
+            uint32_t cw[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) cw[i] = (uint32_t)hw[1 + 2 * i] | ((uint32_t)hw[2 + 2 * i] << 16);
+            LDS unsigned char *krow = Lu + PF_Q8_KC + rq * 256;
+            const u32x4 c0 = {cw[0], cw[1], cw[2], cw[3]}, c1 = {cw[4], cw[5], cw[6], cw[7]};
+            *reinterpret_cast<LDS u32x4 *>(krow + 16u * ((2u * bb) ^ (rq & 15u))) = c0;
+            *reinterpret_cast<LDS u32x4 *>(krow + 16u * ((2u * bb + 1u) ^ (rq & 15u))) = c1;
+            reinterpret_cast<LDS float *>(Lu + PF_Q8_KS)[t] = h2f(hw[0]);
             sched_fence();
             att_q8_split(raw + ATT_Q8_RAWB, Lu + PF_Q8_VC + rq * 256 + 32u * bb,
                          reinterpret_cast<LDS float *>(Lu + PF_Q8_VS) + t);
@@ -491,111 +515,185 @@ __global__ __launch_bounds__(256) void attn_prefill_split_kernel(AttnPrefill a, 
             kt = Lu + PF_Q8_KC;
             vt = Lu + PF_Q8_VC;
         }
-        float part[4 * PF_SLOTS];
+        // scores: rows 16 rb + l16 (A), queries (B); all of the tile's reads first
+        u32x4 kraw[2][2];
+        float ks[2][2];
 #pragma unroll
-        for (uint32_t i = 0; i < 4; i++) {
-            const uint32_t r = rr + 8 * (i ^ (mp >> 3));
-            const LDS unsigned char *kr = kt + r * (Q8 ? 256u : 512u);
-            const float ks = Q8 ? reinterpret_cast<const LDS float *>(Lu + PF_Q8_KS)[r * 8 + (p >> 2)] : 0.0f;
-            float kd[8];
-            att_row8<Q8>(kr, p, ks, kd);
+        for (uint32_t rb = 0; rb < 2; rb++)
 #pragma unroll
-            for (uint32_t s = 0; s < PF_SLOTS; s++) {
-                float d = 0.0f;
+            for (uint32_t jj = 0; jj < 2; jj++) {
+                const uint32_t row = 16 * rb + l16, p = xp + 16 * jj;
+                if constexpr (!Q8) {
+                    kraw[rb][jj] = *reinterpret_cast<const LDS u32x4 *>(kt + row * 512u + 16u * (p ^ l16));
+                } else {
+                    // (8 codes: half p % 2 of 16-byte chunk p / 2, in its slot)
+                    const u32x2 u = *reinterpret_cast<const LDS u32x2 *>(kt + row * 256u + 16u * ((p >> 1) ^ l16) + 8u * (p & 1u));
+                    kraw[rb][jj] = u32x4{u.x, u.y, 0u, 0u};
+                    ks[rb][jj] = reinterpret_cast<const LDS float *>(Lu + PF_Q8_KS)[row * 8 + (p >> 2)];
+                }
+            }
+        sched_fence();
 #pragma unroll
-                for (uint32_t dd = 0; dd < 8; dd++) d = fmaf(qv[s][dd], kd[dd], d);
-                part[i * PF_SLOTS + s] = d;
+        for (uint32_t rb = 0; rb < 2; rb++) {
+            f32x16 d[2];
+#pragma unroll
+            for (uint32_t jj = 0; jj < 2; jj++) {
+                float kd[8];
+#pragma unroll
+                for (uint32_t k = 0; k < 8; k++) {
+                    const uint32_t u = kraw[rb][jj][Q8 ? k >> 2 : k >> 1];
+                    if constexpr (!Q8) kd[k] = h2f((uint16_t)(u >> (16 * (k & 1u))));
+                    else kd[k] = (float)(int)(int8_t)((u >> (8 * (k & 3u))) & 0xffu) * ks[rb][jj];
+                }
+                d[jj] = z16;
+#pragma unroll
+                for (uint32_t dd = 0; dd < 8; dd++)
+                    d[jj] = __builtin_amdgcn_mfma_f32_16x16x1f32(kd[dd], qv[jj][dd], d[jj], 0, 0, 0);
+            }
+            // lane masks 16, 15, 7: elements 4 b + v of both, blocks (0, 1) and (2, 3), the two pairs
+#pragma unroll
+            for (uint32_t v = 0; v < 4; v++) {
+                const float b0 = d[0][v] + d[1][v], b1 = d[0][4 + v] + d[1][4 + v];
+                const float b2 = d[0][8 + v] + d[1][8 + v], b3 = d[0][12 + v] + d[1][12 + v];
+                const float c0 = b0 + b1, c1 = b2 + b3;
+                S[(w * 32 + 16 * rb + 4 * lb + v) * PF_SLOTS + l16] = c0 + c1;
             }
         }
-        att_rs_step_x16(part);
-        att_rs_step<DPP_MIRROR, 8>(part);
-        att_rs_step<DPP_HALF_MIRROR, 4>(part);
-        att_rs_step<DPP_XOR2, 2>(part);
-        att_rs_step<DPP_XOR1, 1>(part);
+        // the V rows of row groups 2w and 2w + 1, read while the scores cross
+        // (f16; the Q8_0 codes and scales where they are used, for registers)
+        u32x2 vraw[4][2];
+        if constexpr (!Q8) {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++)
+#pragma unroll
+                for (uint32_t gi = 0; gi < 2; gi++)
+                    vraw[i][gi] = *reinterpret_cast<const LDS u32x2 *>(vt + (2 * w + gi + 8 * i) * 512u + 8u * lane);
+        }
+        __syncthreads();
+        bool rescale;
         {
-            const uint32_t row = t0 + rr + 8 * my_i;
-            const bool valid = row >= my0 && row < my1;
-            const float sv = valid ? part[0] * a.scale : -INFINITY;
-            float mt = fmaxf(sv, dpp_f<DPP_MIRROR>(sv));
-            mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+            float sv[2], wg[2];
+            bool ok[2];
+#pragma unroll
+            for (uint32_t i = 0; i < 2; i++) {
+                const uint32_t r = rr + 8 * (2 * hf + i), o = r * PF_SLOTS + sq;
+                // lane masks 2, 1
+                const float e0 = S[o] + S[2 * 32 * PF_SLOTS + o], e1 = S[32 * PF_SLOTS + o] + S[3 * 32 * PF_SLOTS + o];
+                ok[i] = t0 + r >= my0 && t0 + r < my1;
+                sv[i] = ok[i] ? (e0 + e1) * a.scale : -INFINITY;
+            }
+            float mt = fmaxf(sv[0], sv[1]);
+            mt = fmaxf(mt, dpp_f<DPP_XOR1>(mt));
             const float mn = fmaxf(mrun, mt);
-            const float wgt = valid ? att_exp(sv - mn) : 0.0f;
-            float ws = wgt + dpp_f<DPP_MIRROR>(wgt);
-            ws = ws + __shfl_xor(ws, 16, 64);
-            const float cf = mrun == -INFINITY ? 0.0f : (mrun == mn ? 1.0f : att_exp(mrun - mn));
+#pragma unroll
+            for (uint32_t i = 0; i < 2; i++) {
+                wg[i] = ok[i] ? att_exp(sv[i] - mn) : 0.0f;
+                W[(rr + 8 * (2 * hf + i)) * PF_SLOTS + sq] = wg[i];
+            }
+            float ws = wg[0] + wg[1];
+            ws = ws + dpp_f<DPP_XOR1>(ws);
+            // the correction is 1 unless the maximum moved, in few tiles
+            float cf = mrun == -INFINITY ? 0.0f : 1.0f;
+            const bool moved = mrun != -INFINITY && mrun != mn;
+            if (__builtin_amdgcn_ballot_w64(moved) != 0) {
+                const float ce = att_exp(mrun - mn);
+                cf = moved ? ce : cf;
+            }
             const float lc = lrun * cf;
             lrun = lc + ws;
             mrun = mn;
-            wgr[my_i * PF_SLOTS + my_s] = wgt;
-            if (my_i == 0) wgr[4 * PF_SLOTS + my_s] = cf;
+            if (hf == 0) CF[rr * PF_SLOTS + sq] = cf;
+            rescale = __builtin_amdgcn_ballot_w64(cf != 1.0f) != 0;
         }
-        // (read back by this wave only: LDS accesses of a wave complete in order)
-        {
-            const f32x4 c0 = *reinterpret_cast<const LDS f32x4 *>(wgr + 4 * PF_SLOTS);
-            const f32x4 c1 = *reinterpret_cast<const LDS f32x4 *>(wgr + 4 * PF_SLOTS + 4);
-            const float cfv[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+        // (weights and corrections are read back by this wave only: LDS
+        // accesses of a wave complete in order)
+        if (rescale) {
 #pragma unroll
-            for (uint32_t s = 0; s < PF_SLOTS; s++)
+            for (uint32_t gi = 0; gi < 2; gi++) {
+                const f32x4 cv = *reinterpret_cast<const LDS f32x4 *>(CF + (2 * w + gi) * PF_SLOTS + 4 * lb);
 #pragma unroll
-                for (uint32_t dd = 0; dd < 8; dd++) acc[s][dd] = acc[s][dd] * cfv[s];
-        }
+                for (uint32_t jj = 0; jj < 4; jj++)
 #pragma unroll
-        for (uint32_t i = 0; i < 4; i++) {
-            const uint32_t r = rr + 8 * i;
-            if (t0 + r < U1) {
-                const LDS unsigned char *vr = vt + r * (Q8 ? 256u : 512u);
-                const float vs = Q8 ? reinterpret_cast<const LDS float *>(Lu + PF_Q8_VS)[r * 8 + (p >> 2)] : 0.0f;
-                float vd[8];
-                att_row8<Q8>(vr, p, vs, vd);
-                const f32x4 w0 = *reinterpret_cast<const LDS f32x4 *>(wgr + i * PF_SLOTS);
-                const f32x4 w1 = *reinterpret_cast<const LDS f32x4 *>(wgr + i * PF_SLOTS + 4);
-                const float w8[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-#pragma unroll
-                for (uint32_t s = 0; s < PF_SLOTS; s++)
-#pragma unroll
-                    for (uint32_t dd = 0; dd < 8; dd++) acc[s][dd] = fmaf(w8[s], vd[dd], acc[s][dd]);
+                    for (uint32_t e = 0; e < 16; e++) acc[gi][jj][e] = acc[gi][jj][e] * cv[e & 3u];
             }
         }
+        float wt[4][2];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++)
+#pragma unroll
+            for (uint32_t gi = 0; gi < 2; gi++) wt[i][gi] = W[(2 * w + gi + 8 * i) * PF_SLOTS + l16];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++)
+#pragma unroll
+            for (uint32_t gi = 0; gi < 2; gi++) {
+                float vd[4];
+                if constexpr (!Q8) {
+                    const u32x2 u = vraw[i][gi];
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; k++) vd[k] = h2f((uint16_t)((k < 2 ? u.x : u.y) >> (16 * (k & 1u))));
+                } else {
+                    const uint32_t r = 2 * w + gi + 8 * i, u = *reinterpret_cast<const LDS uint32_t *>(vt + r * 256u + 4u * lane);
+                    const float vs = reinterpret_cast<const LDS float *>(Lu + PF_Q8_VS)[r * 8 + (lane >> 3)];
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; k++) vd[k] = (float)(int)(int8_t)((u >> (8 * k)) & 0xffu) * vs;
+                }
+#pragma unroll
+                for (uint32_t jj = 0; jj < 4; jj++)
+                    acc[gi][jj] = __builtin_amdgcn_mfma_f32_16x16x1f32(wt[i][gi], vd[jj], acc[gi][jj], 0, 0, 0);
+            }
     }
     // the chunk's partial per query: the eight row groups merged (through
-    // LDS, in the tile region) as the decode merges them
-    LDS float *comb = reinterpret_cast<LDS float *>(Lu);   // [8 rr][8 slots][256]
-    __syncthreads();
-#pragma unroll
-    for (uint32_t s = 0; s < PF_SLOTS; s++) {
-        LDS float *d = comb + (rr * PF_SLOTS + s) * 256 + 8 * p;
-        const f32x4 v0 = {acc[s][0], acc[s][1], acc[s][2], acc[s][3]};
-        const f32x4 v1 = {acc[s][4], acc[s][5], acc[s][6], acc[s][7]};
-        *reinterpret_cast<LDS f32x4 *>(d) = v0;
-        *reinterpret_cast<LDS f32x4 *>(d + 4) = v1;
-    }
-    if (my_i == 0) {
-        gml[rr * PF_SLOTS + my_s] = mrun;
-        gml[8 * PF_SLOTS + rr * PF_SLOTS + my_s] = lrun;
+    // LDS, in the tile region, 8 queries at a time) as the decode merges them
+    LDS float *comb = reinterpret_cast<LDS float *>(Lu);   // [8 groups][8 queries][256]
+    if (hf == 0) {
+        gml[rr * PF_SLOTS + sq] = mrun;
+        gml[(8 + rr) * PF_SLOTS + sq] = lrun;
     }
     __syncthreads();
-    {
-        const uint32_t s = t >> 5, po = t & 31;
-        uint32_t k0, k1;
-        range(s, k0, k1);
+    // each group's weight once (threads 0-127: group t / 16, query t % 16)
+    LDS float *ge = W, *gM = W + 8 * PF_SLOTS;
+    if (t < 8 * PF_SLOTS) {
         float M = -INFINITY;
 #pragma unroll
-        for (uint32_t g2 = 0; g2 < 8; g2++) M = fmaxf(M, gml[g2 * PF_SLOTS + s]);
+        for (uint32_t g2 = 0; g2 < 8; g2++) M = fmaxf(M, gml[g2 * PF_SLOTS + l16]);
+        const float mg = gml[t];
+        ge[t] = mg != -INFINITY ? att_exp(mg - M) : 0.0f;
+        if (t < PF_SLOTS) gM[t] = M;
+    }
+#pragma unroll
+    for (uint32_t qh = 0; qh < 2; qh++) {
+        if (qh) __syncthreads();
+        if (lb >> 1 == qh) {
+#pragma unroll
+            for (uint32_t gi = 0; gi < 2; gi++)
+#pragma unroll
+                for (uint32_t v = 0; v < 4; v++)
+#pragma unroll
+                    for (uint32_t b = 0; b < 4; b++) {
+                        const f32x4 o = {acc[gi][0][4 * b + v], acc[gi][1][4 * b + v], acc[gi][2][4 * b + v],
+                                         acc[gi][3][4 * b + v]};
+                        *reinterpret_cast<LDS f32x4 *>(comb + ((2 * w + gi) * 8 + 4 * (lb & 1u) + v) * 256 + 64 * b +
+                                                       4 * l16) = o;
+                    }
+        }
+        __syncthreads();
+        const uint32_t s = t >> 5, po = t & 31, q = 8 * qh + s;
+        const float M = gM[q];
         float Lc = 0.0f, o[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (uint32_t g2 = 0; g2 < 8; g2++) {
-            const float mg = gml[g2 * PF_SLOTS + s];
-            const float e = mg != -INFINITY ? att_exp(mg - M) : 0.0f;
-            Lc = fmaf(e, gml[8 * PF_SLOTS + g2 * PF_SLOTS + s], Lc);
-            const f32x4 c0 = *reinterpret_cast<const LDS f32x4 *>(comb + (g2 * PF_SLOTS + s) * 256 + 8 * po);
-            const f32x4 c1 = *reinterpret_cast<const LDS f32x4 *>(comb + (g2 * PF_SLOTS + s) * 256 + 8 * po + 4);
+            const float e = ge[g2 * PF_SLOTS + q];
+            Lc = fmaf(e, gml[(8 + g2) * PF_SLOTS + q], Lc);
+            const f32x4 c0 = *reinterpret_cast<const LDS f32x4 *>(comb + (g2 * 8 + s) * 256 + 8 * po);
+            const f32x4 c1 = *reinterpret_cast<const LDS f32x4 *>(comb + (g2 * 8 + s) * 256 + 8 * po + 4);
             const float cv[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
 #pragma unroll
             for (uint32_t dd = 0; dd < 8; dd++) o[dd] = fmaf(e, cv[dd], o[dd]);
         }
-        if (k1 > k0) {
+        const uint32_t m0 = (uint32_t)__shfl((int)k0, (int)q, 64), m1 = (uint32_t)__shfl((int)k1, (int)q, 64);
+        if (m1 > m0) {
             const uint32_t PS = att_rec(HD);
-            float *d = a.part + (((size_t)(q0 + s) * NQ + head) * C + c) * PS;
+            float *d = a.part + (((size_t)(q0 + q) * NQ + head) * C + c) * PS;
             reinterpret_cast<float4 *>(d + 8 * po)[0] = make_float4(o[0], o[1], o[2], o[3]);
             reinterpret_cast<float4 *>(d + 8 * po)[1] = make_float4(o[4], o[5], o[6], o[7]);
             if (po == 0) {
@@ -634,8 +732,17 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(AttnPrefill a) 
     }
     __syncthreads();
     if (t < HD) {
+        // eight chunks' values in flight (past the last: re-read, weight and
+        // add skipped)
         float O = 0.0f;
-        for (uint32_t k = 0; k < NC; k++) O = fmaf(e[k], pb[(size_t)k * PS + t], O);
+        for (uint32_t k = 0; k < NC; k += 8) {
+            float v[8];
+#pragma unroll
+            for (uint32_t i = 0; i < 8; i++) v[i] = pb[(size_t)min(k + i, NC - 1) * PS + t];
+#pragma unroll
+            for (uint32_t i = 0; i < 8; i++)
+                if (k + i < NC) O = fmaf(e[k + i], v[i], O);
+        }
         const float gate = a.qg[((size_t)q * a.nq + head) * 2 * HD + HD + t];
         a.out[((size_t)q * a.nq + head) * HD + t] = (O / Ls) * dev_sigmoid(gate);
     }

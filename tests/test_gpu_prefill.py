@@ -229,3 +229,31 @@ def test_batched_prefill_across_a_change_of_tiles_per_chunk(sn, torch_gpu, past,
     finally:
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("kv", ["f16", "q8_0"])
+@pytest.mark.parametrize("past,chunks,cmin", [(0, 64, 32), (30, 3, 32), (250, 5, 64), (508, 64, 128)])
+def test_batched_prefill_attention_query_blocks(sn, torch_gpu, kv, past, chunks, cmin):
+    """The prefill attention takes 16 queries per item: 1, 15, 16, 17 and 33
+    of them behind a context, at depths where the split's tiles per chunk and
+    chunk count change inside a block, against one pass per token."""
+    cfg = small_config(sn, n_layer=2, n_ctx=past + 96)
+    cfg.attn_every, cfg.attn_chunks, cfg.attn_chunk_min = 1, chunks, cmin
+    cfg.t_kv = sn.Q8_0 if kv == "q8_0" else sn.F16
+    toks = [int(t) for t in np.random.default_rng(past + chunks).integers(0, cfg.n_vocab, 82)]
+    a, b = sn.Model(cfg, seed=57), sn.Model(cfg, seed=57)
+    try:
+        a.synth_context(past, seed=58)
+        b.synth_context(past, seed=58)
+        pos, i = past, 0
+        for n in (1, 15, 16, 17, 33):
+            print(f"attention blocks kv={kv} past={past} chunks={chunks}: {n} tokens at {pos}", flush=True)
+            nxt_a = a.prefill(toks[i:i + n], pos, mode="batched")
+            nxt_b = b.prefill(toks[i:i + n], pos, mode="tokenwise")
+            pos, i = pos + n, i + n
+            assert nxt_a == nxt_b
+            assert np.array_equal(a.logits(), b.logits())
+            same_state(a, b, cfg)
+    finally:
+        a.close()
+        b.close()
