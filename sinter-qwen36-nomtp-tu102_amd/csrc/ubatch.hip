@@ -425,10 +425,12 @@ __global__ __launch_bounds__(UB_THREADS, 2) void ubatch_gemm_kernel(UbArgs a) {
 // KW, ...), each wave's weights and activations straight from memory, so the
 // loads of a whole row are in flight at once.  The terms of a round of KW
 // items meet in LDS (double-buffered), where each (row, token) is folded by
-// one thread in item order.
+// one thread in item order.  One token tile is held to 128 registers, four
+// workgroups on a CU instead of three: Q6_K 248320 x 5120, 1 token 262 -> 244 us,
+// Q4_K 12416 x 5120 15.0 -> 13.5 (eight waves of a workgroup to the items: 15.4).
 constexpr uint32_t UB_KW = 4;
 template <int WT, uint32_t NT>
-__global__ __launch_bounds__(64 * UB_KW) void ubatch_gemv_kernel(UbArgs a) {
+__global__ __launch_bounds__(64 * UB_KW, NT == 1 ? 4 : 2) void ubatch_gemv_kernel(UbArgs a) {
     constexpr uint32_t KW = UB_KW, OUT = NT * UB_TOK * UB_ROWS, THREADS = 64u * KW, PT = (OUT + THREADS - 1u) / THREADS;
     __shared__ double terms[2][KW][OUT];
     LDS double *T = (LDS double *)terms;
@@ -735,9 +737,11 @@ struct UbSplit {
 //   many-token kernel: up to one workgroup per CU it runs at its latency
 //   `lone`; with w > 1 per CU the CU's issue slots bound it, `thr` per
 //   workgroup, and a started last round takes about two thirds of one;
-//   few-token kernel: latency, or `thr` per workgroup of a CU over a start-up.
+//   few-token kernel: latency, or `thr` per workgroup of a CU over a start-up;
+//   each further token's activations are another line of a load.
 // E.g. Q6_K 5120 x 17408 at 256 tokens (us): nt 2 180, 3 131, 4 143, 6 118,
-// 8 143; at 8 tokens few-token 39, many-token 86.  Q4_K 34816 x 5120 at 256:
+// 8 143; at 5 tokens few-token 37, many-token 90; 151936 x 5120 at 1, 5 and 16
+// tokens: few-token 154, 162, 193, many-token 175, 186, 195.  Q4_K 34816 x 5120 at 256:
 // nt 2 205, 4 180, 6 181, 8 166; 8192 x 5120 at 24: few-token 15, nt 1 15.5.
 template <int WT>
 UbSplit ub_split(const UbArgs &a) {
@@ -762,7 +766,8 @@ UbSplit ub_split(const UbArgs &a) {
     };
     // (not compiled, as never the cheapest: few-token nt 2 for Q4_K, whose
     // unpacking is cheap enough to repeat; many-token nt 1 for Q6_K, whose is not)
-    consider(true, 1, Q4 ? 370 : 560, Q4 ? 166 : 250, Q4 ? 200 : 150);
+    const uint32_t tok = std::min(a.n_tok, UB_TOK);
+    consider(true, 1, Q4 ? 370 : 560, Q4 ? 166 : 200 + 3 * tok, Q4 ? 200 : 150);
     if (!Q4 && tiles > 1) consider(true, 2, 700, 420, 150);
     if (a.nb > UB_MAX_NB) return best;
     for (uint32_t nt : {Q4 ? 1u : 2u, 2u, 3u, 4u, 6u, 8u})
