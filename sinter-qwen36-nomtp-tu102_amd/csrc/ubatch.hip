@@ -524,25 +524,27 @@ __global__ __launch_bounds__(64 * UB_KW, NT == 1 ? 4 : 2) void ubatch_gemv_kerne
 // ggml quantize_row_q8_K_ref over a ubatch (the oracle's or_quant_q8_K):
 // one wave per 256-element block, lane l holding elements 4l..4l+3.  The
 // block's scale comes from its first element of largest |x| (sequentially:
-// `if (|x| > amax)`, so a tie keeps the lower index -- the wave reduction
-// breaks ties by index), iscale = -127 / that element, codes
+// `if (|x| > amax)`, so a tie keeps the lower index: that of the
+// first lane with the wave's maximum), iscale = -127 / that element, codes
 // min(127, rint(iscale * x)) (ggml's nearest_int: round half to even), d =
 // 1 / iscale, bsums the 16-element sums of the codes; an all-zero block is
 // all zeros.  Inputs are finite.
 __device__ __forceinline__ void quant_block_q8k(const float e[4], uint32_t lane, uint8_t *ob) {
     float amax = 0.0f, mx = 0.0f;
-    uint32_t idx = 0xFFFFFFFFu;
 #pragma unroll
     for (uint32_t j = 0; j < 4; j++) {
         const float ax = fabsf(e[j]);
-        if (ax > amax) { amax = ax; mx = e[j]; idx = 4u * lane + j; }
+        if (ax > amax) { amax = ax; mx = e[j]; }
     }
-#pragma unroll
-    for (uint32_t o = 1; o < 64; o <<= 1) {
-        const float a2 = __shfl_xor(amax, o), m2 = __shfl_xor(mx, o);
-        const uint32_t i2 = __shfl_xor(idx, o);
-        if (a2 > amax || (a2 == amax && i2 < idx)) { amax = a2; mx = m2; idx = i2; }
-    }
+    // (by DPP, readlanes and a ballot: a chain of 18 LDS shuffles of (|x|, x,
+    // index) took longer than the rest of the block)
+    auto lane_f = [](float v, uint32_t l) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), (int)l));
+    };
+    const float rm = row16_max(amax);
+    const float wm = fmaxf(fmaxf(lane_f(rm, 0), lane_f(rm, 16)), fmaxf(lane_f(rm, 32), lane_f(rm, 48)));
+    mx = lane_f(mx, (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(amax == wm)));
+    amax = wm;
     int q[4] = {0, 0, 0, 0};
     float d = 0.0f;
     if (amax != 0.0f) {
@@ -557,8 +559,8 @@ __device__ __forceinline__ void quant_block_q8k(const float e[4], uint32_t lane,
     *(uint32_t *)(ob + 4u + 4u * lane) =
         (uint32_t)(q[0] & 0xFF) | ((uint32_t)(q[1] & 0xFF) << 8) | ((uint32_t)(q[2] & 0xFF) << 16) | ((uint32_t)q[3] << 24);
     int bs = q[0] + q[1] + q[2] + q[3];
-    bs += __shfl_xor(bs, 1);
-    bs += __shfl_xor(bs, 2);
+    bs += dpp_i<DPP_XOR1>(bs);
+    bs += dpp_i<DPP_XOR2>(bs);
     if ((lane & 3u) == 0) *(int16_t *)(ob + 260u + 2u * (lane >> 2)) = (int16_t)bs;
     if (lane == 0) *(float *)ob = d;
 }
@@ -677,43 +679,72 @@ __global__ __launch_bounds__(256) void conv_state_kernel(const float *__restrict
 // four partial sums (element i into sum i / 4) over its chunks g + 32,
 // g + 48, ... and then g and g + 16; the row adds them as
 // (s0 + s1) + (s2 + s3) and by its DPP butterfly, the wave its four rows in
-// order, the workgroup its four waves in order.  Then wave v quantises
-// blocks v, v + 4, ... of the normalised row.
-__device__ __forceinline__ void ub_add_sq(const float *xr, uint32_t c, uint32_t r, double s4[4]) {
+// order, the workgroup its four waves in order.  Those are the first four
+// waves; the normalised row is quantised by up to 16, wave v blocks v,
+// v + 16, ..., the first two of them loaded before the sum: a token is one
+// chain of latencies (four waves with each block's load behind the sum: 9.1
+// us at K 5120, 24 tokens, 5.0 us so).
+constexpr uint32_t UB_NORM_WAVES = 16;
+__device__ __forceinline__ void ub_add_sq(const float4 x[4], double s4[4]) {
 #pragma unroll
     for (uint32_t q = 0; q < 4; q++) {
-        const float4 v = ((const float4 *)(xr + 256u * c + 16u * r))[q];
-        s4[q] += (double)(v.x * v.x);
-        s4[q] += (double)(v.y * v.y);
-        s4[q] += (double)(v.z * v.z);
-        s4[q] += (double)(v.w * v.w);
+        s4[q] += (double)(x[q].x * x[q].x);
+        s4[q] += (double)(x[q].y * x[q].y);
+        s4[q] += (double)(x[q].z * x[q].z);
+        s4[q] += (double)(x[q].w * x[q].w);
     }
 }
-__global__ __launch_bounds__(256) void rmsnorm_quant_q8k_kernel(const float *__restrict__ x, const float *__restrict__ w,
-                                                               float eps, uint32_t k, uint8_t *__restrict__ xq) {
+__global__ __launch_bounds__(64 * UB_NORM_WAVES) void rmsnorm_quant_q8k_kernel(const float *__restrict__ x,
+                                                                              const float *__restrict__ w, float eps,
+                                                                              uint32_t k, uint8_t *__restrict__ xq) {
     __shared__ double red[4];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6, r = tid & 15u, g = tid >> 4, nchunk = k / 256u;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, r = tid & 15u, g = tid >> 4, nchunk = k / 256u;
+    const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const float *xr = x + (size_t)blockIdx.x * k;
-    double s4[4] = {0.0, 0.0, 0.0, 0.0};
-    for (uint32_t c = g + 32u; c < nchunk; c += 16u) ub_add_sq(xr, c, r, s4);
-    if (g < nchunk) ub_add_sq(xr, g, r, s4);
-    if (g + 16u < nchunk) ub_add_sq(xr, g + 16u, r, s4);
-    double s = row16_sum_f64((s4[0] + s4[1]) + (s4[2] + s4[3]));
-    s = ((readlane_f64(s, 0) + readlane_f64(s, 16)) + readlane_f64(s, 32)) + readlane_f64(s, 48);
-    if (lane == 0) red[wv] = s;
+    auto chunk = [&](uint32_t c, float4 v[4]) {   // the lane's elements of chunk c (past the last: the last's)
+#pragma unroll
+        for (uint32_t q = 0; q < 4; q++) v[q] = ((const float4 *)(xr + 256u * min(c, nchunk - 1u) + 16u * r))[q];
+    };
+    float4 a[4], b[4], xv[2], gv[2];
+    if (wv < 4u) {
+        chunk(g, a);
+        chunk(g + 16u, b);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 2; j++) {
+        const uint32_t bl = min(wv + UB_NORM_WAVES * j, nchunk - 1u);
+        xv[j] = ((const float4 *)(xr + 256u * bl))[lane];
+        gv[j] = w ? ((const float4 *)(w + 256u * bl))[lane] : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+    }
+    if (wv < 4u) {
+        double s4[4] = {0.0, 0.0, 0.0, 0.0};
+        for (uint32_t c = g + 32u; c < nchunk; c += 16u) {
+            float4 v[4];
+            chunk(c, v);
+            ub_add_sq(v, s4);
+        }
+        if (g < nchunk) ub_add_sq(a, s4);
+        if (g + 16u < nchunk) ub_add_sq(b, s4);
+        double s = row16_sum_f64((s4[0] + s4[1]) + (s4[2] + s4[3]));
+        s = ((readlane_f64(s, 0) + readlane_f64(s, 16)) + readlane_f64(s, 32)) + readlane_f64(s, 48);
+        if (lane == 0) red[wv] = s;
+    }
     __syncthreads();
-    s = ((red[0] + red[1]) + red[2]) + red[3];
+    const double s = ((red[0] + red[1]) + red[2]) + red[3];
     const float mean = (float)(s / (double)k);
     const float scale = 1.0f / sqrtf(mean + eps);
-    uint8_t *orow = xq + (size_t)blockIdx.x * (k / 256u) * Q8K_BYTES;
-    for (uint32_t b = wv; b < k / 256u; b += 4u) {
-        const float4 v = ((const float4 *)(xr + 256u * b))[lane];
+    uint8_t *orow = xq + (size_t)blockIdx.x * nchunk * Q8K_BYTES;
+    auto quant = [&](uint32_t bl, const float4 &v, const float4 &gm) {
         float e[4] = {v.x * scale, v.y * scale, v.z * scale, v.w * scale};
-        if (w) {
-            const float4 g = ((const float4 *)(w + 256u * b))[lane];
-            e[0] = e[0] * g.x; e[1] = e[1] * g.y; e[2] = e[2] * g.z; e[3] = e[3] * g.w;
-        }
-        quant_block_q8k(e, lane, orow + (size_t)b * Q8K_BYTES);
+        if (w) { e[0] = e[0] * gm.x; e[1] = e[1] * gm.y; e[2] = e[2] * gm.z; e[3] = e[3] * gm.w; }
+        quant_block_q8k(e, lane, orow + (size_t)bl * Q8K_BYTES);
+    };
+#pragma unroll
+    for (uint32_t j = 0; j < 2; j++)
+        if (wv + UB_NORM_WAVES * j < nchunk) quant(wv + UB_NORM_WAVES * j, xv[j], gv[j]);
+    for (uint32_t bl = wv + 2u * UB_NORM_WAVES; bl < nchunk; bl += UB_NORM_WAVES) {
+        const float4 v = ((const float4 *)(xr + 256u * bl))[lane];
+        quant(bl, v, w ? ((const float4 *)(w + 256u * bl))[lane] : v);
     }
 }
 
@@ -878,7 +909,7 @@ extern "C" int sinter_rmsnorm_quant_q8k_ubatch(const float *x, const float *w, f
     if ((uintptr_t)x % 16u || (uintptr_t)w % 16u || (uintptr_t)xq % 4u)
         return set_error(SINTER_ERR_ARG, "rmsnorm_quant_q8k_ubatch: alignment (x, w 16 bytes, xq 4 bytes)");
     if (!(eps >= 0.0f)) return set_error(SINTER_ERR_ARG, "rmsnorm_quant_q8k_ubatch: eps must be >= 0");
-    hipLaunchKernelGGL(rmsnorm_quant_q8k_kernel, dim3(n_tokens), dim3(256), 0, (hipStream_t)stream, x, w, eps,
+    hipLaunchKernelGGL(rmsnorm_quant_q8k_kernel, dim3(n_tokens), dim3(64 * UB_NORM_WAVES), 0, (hipStream_t)stream, x, w, eps,
                        (uint32_t)k, (uint8_t *)xq);
     return hip_ok(hipGetLastError(), "rmsnorm_quant_q8k_ubatch: launch") ? SINTER_OK : SINTER_ERR_HIP;
 }

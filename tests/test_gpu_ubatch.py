@@ -316,3 +316,31 @@ def test_conv_silu_ubatch_matches_oracle_token_loop(sn, orc, torch_gpu, channels
         assert np.array_equal(got[t], out), t
     if dconv > 1:
         assert np.array_equal(host(dst), ref_st)
+
+
+@pytest.mark.parametrize("k", [256, 3840, 4096, 4352, 8192, 8448, 16640])
+def test_rmsnorm_quant_q8k_ubatch_chunk_edges(sn, orc, torch_gpu, k):
+    """Rows of 1, 15, 16, 17, 32, 33 and 65 blocks: a wave quantises blocks v,
+    v + 16 and, past 32, further ones; the sum's groups hold 0 to 5 chunks."""
+    test_rmsnorm_quant_q8k_ubatch_matches_oracle(sn, orc, torch_gpu, k, 3, True)
+
+
+def test_quant_q8k_ubatch_ties(sn, orc, torch_gpu):
+    """The block's scale takes the sign of the first element of largest
+    magnitude, wherever in the wave the ties lie."""
+    torch = torch_gpu
+    rng = np.random.default_rng(11)
+    x = rng.uniform(-1, 1, (64, 256)).astype(np.float32)
+    for b in range(64):
+        at = rng.choice(256, 2 + b % 5, replace=False)
+        x[b, at] = np.where(rng.random(at.size) < 0.5, -2.0, 2.0)
+    x[0] = 0.0
+    x[1] = -3.0
+    dx, dq = dev(torch, x.reshape(-1)), torch.empty(64 * 292, dtype=torch.uint8, device="cuda")
+    print("quant_q8k_ubatch ties", flush=True)
+    sn.check(sn.lib().sinter_quant_q8k_ubatch(C.c_void_p(dx.data_ptr()), 256, 64, C.c_void_p(dq.data_ptr()),
+                                              C.c_void_p(stream(torch))), "quant")
+    torch.cuda.synchronize()
+    want = np.empty(64 * 292, np.uint8)
+    orc.lib().or_quant_q8_K(x.ctypes.data, want.ctypes.data, x.size)
+    assert np.array_equal(host(dq), want)
