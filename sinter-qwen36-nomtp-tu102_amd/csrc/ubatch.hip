@@ -620,53 +620,50 @@ __global__ __launch_bounds__(64) void gated_norm_quant_q8k_kernel(const float *_
 // st[c][nh + tau] for -nh <= tau < 0 (nh = dconv - 1, oldest first),
 // y[t][c] = silu(sum_j input(t - nh + j) * w[c][j]), the sum in fp64 in tap
 // order rounded once.  Outputs do not depend on each other, so a thread
-// takes channel c over UB_CONV_TOK consecutive tokens (blockIdx.y), its
-// window in registers; the state moves on in conv_state_kernel, launched
-// after this one.
+// takes channel c over UB_CONV_TOK consecutive tokens (blockIdx.y), all their
+// inputs loaded before the first sum.  The state moves on to the last nh
+// inputs (old entries when the ubatch is shorter than nh) in the threads of
+// the first tokens, the only ones that read it: UB_CONV_TOK >= nh.  8192
+// channels, 4 taps: with loads inside the token loop and a second launch for
+// the state 6.9 + 4.7 us at 24 tokens, 11.7 + 4.7 at 256; 4.8 and 7.5 so (7.4
+// and 11.9 with the tap count a variable, whose branches keep a token's taps
+// and the exponentials of different tokens apart).
 constexpr uint32_t UB_CONV_TOK = 8;
-__global__ __launch_bounds__(256) void conv_silu_kernel(const float *__restrict__ x, const float *__restrict__ st,
+static_assert(UB_CONV_TOK >= UB_CONV_MAX - 1, "only a channel's first thread reads the conv state");
+template <uint32_t DC>   // taps
+__global__ __launch_bounds__(256) void conv_silu_kernel(const float *__restrict__ x, float *__restrict__ st,
                                                        const float *__restrict__ cw, float *__restrict__ y,
-                                                       uint32_t channels, uint32_t dconv, uint32_t n_tok) {
+                                                       uint32_t channels, uint32_t n_tok) {
+    constexpr uint32_t NH = DC - 1;
     const uint32_t c = blockIdx.x * 256u + threadIdx.x;
     if (c >= channels) return;
-    const uint32_t nh = dconv - 1u, t0 = blockIdx.y * UB_CONV_TOK, t1 = min(t0 + UB_CONV_TOK, n_tok);
-    float win[UB_CONV_MAX];
-    float wt[UB_CONV_MAX];
+    const uint32_t t0 = blockIdx.y * UB_CONV_TOK;
+    // input(tau), past the ubatch its last token's
+    auto input = [&](int tau) {
+        return tau >= 0 ? x[(size_t)min((uint32_t)tau, n_tok - 1u) * channels + c]
+                        : st[(size_t)c * NH + (uint32_t)(tau + (int)NH)];
+    };
+    float in[NH + UB_CONV_TOK];   // inputs t0 - NH ..
+    double wt[DC];
 #pragma unroll
-    for (uint32_t j = 0; j < UB_CONV_MAX; j++) {
-        const int tau = (int)t0 - (int)nh + (int)j;
-        win[j] = j >= nh ? 0.0f : tau >= 0 ? x[(size_t)tau * channels + c] : st[(size_t)c * nh + (uint32_t)(tau + (int)nh)];
-        wt[j] = j < dconv ? cw[(size_t)c * dconv + j] : 0.0f;
-    }
-    for (uint32_t t = t0; t < t1; t++) {
-        const float xn = x[(size_t)t * channels + c];
+    for (uint32_t j = 0; j < NH + UB_CONV_TOK; j++) in[j] = input((int)(t0 + j) - (int)NH);
+#pragma unroll
+    for (uint32_t j = 0; j < DC; j++) wt[j] = (double)cw[(size_t)c * DC + j];
+#pragma unroll
+    for (uint32_t i = 0; i < UB_CONV_TOK; i++) {
+        if (t0 + i >= n_tok) break;
         double acc = 0.0;
 #pragma unroll
-        for (uint32_t j = 0; j < UB_CONV_MAX; j++)
-            if (j < dconv) acc += (double)(j < nh ? win[j] : xn) * (double)wt[j];
-        y[(size_t)t * channels + c] = dev_silu((float)acc);
-#pragma unroll
-        for (uint32_t j = 0; j + 1 < UB_CONV_MAX; j++)
-            if (j < nh) win[j] = (j + 1 < nh) ? win[j + 1] : xn;
+        for (uint32_t j = 0; j < DC; j++) acc += (double)in[i + j] * wt[j];
+        y[(size_t)(t0 + i) * channels + c] = dev_silu((float)acc);
     }
-}
-
-// The conv state after the ubatch: st[c][j] = input(n_tok - nh + j), the last
-// nh inputs (old state entries when the ubatch is shorter than nh).
-__global__ __launch_bounds__(256) void conv_state_kernel(const float *__restrict__ x, float *__restrict__ st,
-                                                        uint32_t channels, uint32_t dconv, uint32_t n_tok) {
-    const uint32_t c = blockIdx.x * 256u + threadIdx.x;
-    if (c >= channels) return;
-    const uint32_t nh = dconv - 1u;
-    float nv[UB_CONV_MAX];
+    if (t0 == 0) {
+        float nv[NH + 1];
 #pragma unroll
-    for (uint32_t j = 0; j < UB_CONV_MAX; j++) {
-        const int tau = (int)n_tok - (int)nh + (int)j;
-        nv[j] = j >= nh ? 0.0f : tau >= 0 ? x[(size_t)tau * channels + c] : st[(size_t)c * nh + (uint32_t)(tau + (int)nh)];
+        for (uint32_t j = 0; j < NH; j++) nv[j] = input((int)n_tok - (int)NH + (int)j);
+#pragma unroll
+        for (uint32_t j = 0; j < NH; j++) st[(size_t)c * NH + j] = nv[j];
     }
-#pragma unroll
-    for (uint32_t j = 0; j < UB_CONV_MAX; j++)
-        if (j < nh) st[(size_t)c * nh + j] = nv[j];
 }
 
 // RMSNorm then the Q8_K quantiser, one workgroup per token: the norm of the
@@ -959,10 +956,20 @@ extern "C" int sinter_conv_silu_ubatch(const float *x, float *state, const float
     if ((uintptr_t)x % 4u || (uintptr_t)state % 4u || (uintptr_t)conv_w % 4u || (uintptr_t)y % 4u)
         return set_error(SINTER_ERR_ARG, "conv_silu_ubatch: alignment (4 bytes)");
     const uint32_t nblk = (uint32_t)((channels + 255) / 256);
-    hipLaunchKernelGGL(conv_silu_kernel, dim3(nblk, (n_tokens + UB_CONV_TOK - 1) / UB_CONV_TOK), dim3(256), 0,
-                       (hipStream_t)stream, x, state, conv_w, y, (uint32_t)channels, dconv, n_tokens);
-    if (dconv > 1)
-        hipLaunchKernelGGL(conv_state_kernel, dim3(nblk), dim3(256), 0, (hipStream_t)stream, x, state,
-                           (uint32_t)channels, dconv, n_tokens);
+    const dim3 grid(nblk, (n_tokens + UB_CONV_TOK - 1) / UB_CONV_TOK);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, x, state, conv_w, y, (uint32_t)channels,
+                           n_tokens);
+    };
+    switch (dconv) {
+        case 1: launch(conv_silu_kernel<1>); break;
+        case 2: launch(conv_silu_kernel<2>); break;
+        case 3: launch(conv_silu_kernel<3>); break;
+        case 4: launch(conv_silu_kernel<4>); break;
+        case 5: launch(conv_silu_kernel<5>); break;
+        case 6: launch(conv_silu_kernel<6>); break;
+        case 7: launch(conv_silu_kernel<7>); break;
+        default: launch(conv_silu_kernel<8>); break;
+    }
     return hip_ok(hipGetLastError(), "conv_silu_ubatch: launch") ? SINTER_OK : SINTER_ERR_HIP;
 }

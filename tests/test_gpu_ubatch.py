@@ -344,3 +344,11 @@ def test_quant_q8k_ubatch_ties(sn, orc, torch_gpu):
     want = np.empty(64 * 292, np.uint8)
     orc.lib().or_quant_q8_K(x.ctypes.data, want.ctypes.data, x.size)
     assert np.array_equal(host(dq), want)
+
+
+@pytest.mark.parametrize("dconv,n_tok", [(4, 1), (4, 2), (4, 3), (4, 8), (4, 9), (8, 5), (8, 7), (8, 8), (8, 17),
+                                         (3, 4), (5, 10), (6, 16), (7, 6)])
+def test_conv_silu_ubatch_token_edges(sn, orc, torch_gpu, dconv, n_tok):
+    """Ubatches shorter than the conv's history (old state entries move up) and
+    around a thread's eight tokens, for every tap count, channels off 256."""
+    test_conv_silu_ubatch_matches_oracle_token_loop(sn, orc, torch_gpu, 300, dconv, n_tok)
