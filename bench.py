@@ -299,6 +299,7 @@ def ubatch_bench(args):
         blk = np.zeros((T * nb, 292), np.uint8)
         blk[:, 0:4] = (np.abs(rng.standard_normal((T * nb, 1))) * 0.01 + 1e-3).astype(np.float32).view(np.uint8)
         blk[:, 4:260] = rng.integers(-127, 128, (T * nb, 256)).astype(np.int8).view(np.uint8)
+        blk[:, 260:292] = blk[:, 4:260].view(np.int8).reshape(-1, 16, 16).sum(2, dtype=np.int16).view(np.uint8)
         xq[k] = torch.from_numpy(blk.reshape(-1)).cuda()
     ys = [torch.empty(T * r, dtype=torch.float32, device="cuda") for _, _, r, _ in UBATCH_MATS]
 
