@@ -93,8 +93,9 @@ __global__ __launch_bounds__(256) void gdn_prep_ubatch_kernel(GdnUb a) {
 // update in the same fp32 expressions.  The state stays in registers from the
 // first token to the last.
 //
-// A token is a dependent chain (kv sum -> delta -> update -> sums) of 7 RPT
-// instructions, one wave's own issue rate: what else a token waits for decides
+// A token is 7 RPT instructions of one wave's own issue (per row the decay, the
+// update's product and sum, two products and two running sums), and the next
+// token's update waits for this one's sums: what else a token waits for decides
 // the time.  k and q come by LDS-DMA, GDN_STAGE tokens at a time and one stage
 // ahead, in the order the lanes read them -- position j TPC + p holds rows
 // RPT p + 4j .. + 3, so the TPC threads of a column read consecutive 16-byte
@@ -127,11 +128,11 @@ __global__ __launch_bounds__(64) void gdn_scan_ubatch_kernel(GdnUb a) {
         const f32x4 t = *reinterpret_cast<const f32x4 *>(srow + r);
         s[r] = t.x; s[r + 1] = t.y; s[r + 2] = t.z; s[r + 3] = t.w;
     }
-    // stage st's inputs: k | q of its tokens into buffer st & 1, v of the
+    // stage st's inputs: k | q of its tokens into buffer `buf`, v of the
     // lane's column, g and beta of token lane % GDN_STAGE in registers
     // (tokens past the last repeat it, never used)
     struct Small { float v[GDN_STAGE], g, b; };
-    auto issue = [&](uint32_t st, Small &w) {
+    auto issue = [&](uint32_t st, uint32_t buf, Small &w) {
         const uint32_t tb = st * GDN_STAGE;
 #pragma unroll
         for (uint32_t i = 0; i < BUF / 1024u; i++) {
@@ -139,7 +140,7 @@ __global__ __launch_bounds__(64) void gdn_scan_ubatch_kernel(GdnUb a) {
             const uint32_t t = min(tb + tk, last), c = (pos % TPC) * (RPT / 4) + pos / TPC;
             // (byte offset from the first token: kn follows qn in one buffer)
             const uint32_t voff = (((half ? 0u : n) + t) * HK + hk) * VEC + 16u * c;
-            lds_dma16<false>((uintptr_t)a.qn, voff, lbase + (st & 1u) * BUF + 1024u * i);
+            lds_dma16<false>((uintptr_t)a.qn, voff, lbase + buf * BUF + 1024u * i);
         }
         const uint32_t tg = min(tb + lane % GDN_STAGE, last);
         w.g = a.gate[(size_t)tg * HV + h];
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(64) void gdn_scan_ubatch_kernel(GdnUb a) {
     auto qvec = [&](uint32_t st, uint32_t i) { return L + (st & 1u) * BUF + i * 2u * VEC + VEC; };
     const uint32_t nst = (n + GDN_STAGE - 1) / GDN_STAGE;
     Small cur, nxt;
-    issue(0, cur);
+    issue(0, 0, cur);
     landed(cur);
     float kc[RPT], qc[RPT], kn[RPT];
     load(kvec(0, 0), kc);
@@ -196,11 +197,12 @@ __global__ __launch_bounds__(64) void gdn_scan_ubatch_kernel(GdnUb a) {
     // whole stages (kc, qc of the stage's first token and kn of the one after
     // it are loaded, dkv is the first token's)
     for (; (st + 1) * GDN_STAGE <= n; st++) {
-        // its buffer was last read in the stage before; the reads still in
-        // flight are at most the last token's prefetch, from the other buffer
-        // (LDS reads complete in order)
-        asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(RPT / 2 < 15 ? RPT / 2 : 15) : "memory");
-        issue(min(st + 1, nst - 1), nxt);
+        // every LDS read so far has landed, the last ones of the buffer that
+        // is filled next among them, in whatever order they were issued (the
+        // last stage fills it too, with its own tokens, which nothing uses: a
+        // branch here cost 6 % at 1024 tokens, 27 % at head size 256)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        issue(min(st + 1, nst - 1), (st + 1) & 1u, nxt);
         const uint32_t tb = st * GDN_STAGE;
         float ov = 0.0f;   // token tb + p's output (every thread of a column has it: one store per stage)
 #pragma unroll
@@ -231,7 +233,6 @@ __global__ __launch_bounds__(64) void gdn_scan_ubatch_kernel(GdnUb a) {
 #pragma unroll
         for (uint32_t r = 0; r < RPT; r++) { kc[r] = kn[r]; qc[r] = qx[r]; kn[r] = kx[r]; }
     }
-    dma_wait();   // (the last staging must not outlive the wave's LDS)
 #pragma unroll
     for (uint32_t r = 0; r < RPT; r += 4) {
         const f32x4 v = {s[r], s[r + 1], s[r + 2], s[r + 3]};
