@@ -40,8 +40,9 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef unsigned short us2 __attribute__((ext_vector_type(2)));
 typedef double v2d __attribute__((ext_vector_type(2)));
-// 16 bytes at a 4-byte boundary (one global_load_dwordx4)
+// 16 bytes at a 4-byte boundary (one global_load_dwordx4), 4 at a 2-byte one
 typedef struct __attribute__((packed, aligned(4))) { uint32_t d[4]; } u128_a4;
+typedef struct __attribute__((packed, aligned(2))) { uint32_t d; } u32_a2;
 
 constexpr uint32_t UB_TOK = 16;      // tokens per tile: the MFMA's M
 constexpr uint32_t UB_ROWS = 16;     // rows per wave: the MFMA's N
@@ -88,7 +89,7 @@ struct WItem<SINTER_Q4_K> {
     static __device__ __forceinline__ uint32_t chunk(uint32_t m, uint32_t g) {
         return 8u * (m >> 1) + 4u * (g >> 1) + 2u * (m & 1u) + (g & 1u);
     }
-    __device__ __forceinline__ void load(const uint8_t *b, uint32_t g) {
+    __host__ __device__ __forceinline__ void load(const uint8_t *b, uint32_t g) {
         const uint4 hv = *(const uint4 *)b;
         h[0] = hv.x; h[1] = hv.y; h[2] = hv.z; h[3] = hv.w;
 #pragma unroll
@@ -137,9 +138,12 @@ struct WItem<SINTER_Q6_K> {
     // CU: 586 cycles at 2 bytes past a boundary, 160 at 4 or 8): each field is
     // loaded from the 4-aligned address at or before it and shifted into place
     // with the dword that follows, which is another lane's first (a load of
-    // its own would take as long as the 16 bytes).  No read leaves the
-    // 4-aligned span of the block.
-    __device__ __forceinline__ void load(const uint8_t *b, uint32_t g) {
+    // its own would take as long as the 16 bytes).  The last dword is the
+    // block's own last four bytes, off a 4-byte boundary where the block is on
+    // one: a read on past the block's end would pass the end of a matrix of an
+    // odd number of blocks (no slower: Q6_K 151936 x 5120, 1 token 153.3 ->
+    // 152.2 us, 5120 x 17408, 256 tokens 117.9 -> 117.4).
+    __host__ __device__ __forceinline__ void load(const uint8_t *b, uint32_t g) {
         sh = (uint32_t)((uintptr_t)b & 3u);
         b -= sh;
 #pragma unroll
@@ -149,10 +153,10 @@ struct WItem<SINTER_Q6_K> {
 #pragma unroll
             for (uint32_t j = 0; j < 4; j++) { l[4 * n + j] = x.d[j]; hq[4 * n + j] = y.d[j]; }
         }
-        const u128_a4 s = *(const u128_a4 *)(b + 192u);   // the scales, then d
+        const u128_a4 s = *(const u128_a4 *)(b + 192u);   // the scales
 #pragma unroll
         for (uint32_t j = 0; j < 4; j++) sc[j] = s.d[j];
-        sc[4] = *(const uint32_t *)(b + 208u);
+        sc[4] = ((const u32_a2 *)(b + sh + 206u))->d;   // the last two scales, d
     }
     __device__ __forceinline__ void unpack(BItem &b, uint32_t g) const {
         const uint32_t f = 2u * (g >> 1);   // the lane's qh field of a nibble: bits f, f + 1 (low), f + 4, f + 5 (high)
@@ -193,8 +197,7 @@ struct WItem<SINTER_Q6_K> {
                 }
             }
         }
-        const uint32_t d = (sc[4] >> (8u * sh)) & 0xFFFFu;
-        b.dw = f16_bits_to_f32(d);
+        b.dw = f16_bits_to_f32(sc[4] >> 16);
         b.dmin = 0.0f;
     }
 };

@@ -1,0 +1,63 @@
+"""The host-computable parts of the batched GEMV (csrc/ubatch.hip), compiled
+for the CPU: which bytes a weight item's loads depend on (no GPU)."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG = os.path.join(ROOT, "sinter-qwen36-nomtp-tu102_amd")
+
+SRC = r"""
+#include "ubatch.hip"
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <new>
+using namespace sinter;
+
+// whether loading item i of n consecutive blocks depends on bytes around them
+template <int WT>
+static bool reads_outside(uint32_t n, uint32_t i, uint32_t g) {
+    typedef WItem<WT> Item;
+    alignas(16) unsigned char buf[2][64 + 8 * 210 + 64], item[2][sizeof(Item)];
+    for (int p = 0; p < 2; p++) {
+        memset(buf[p], p ? 0x5A : 0xA5, sizeof buf[p]);
+        for (uint32_t k = 0; k < n * Item::BYTES; k++) buf[p][64 + k] = (unsigned char)(k * 37u + 11u);
+        // (the object's representation, padding included)
+        memset(item[p], 0, sizeof item[p]);
+        Item *w = new (item[p]) Item;
+        w->load(buf[p] + 64 + i * Item::BYTES, g);
+    }
+    return memcmp(item[0], item[1], sizeof(Item)) != 0;
+}
+
+int main() {
+    for (uint32_t n = 1; n <= 8; n++)
+        for (uint32_t i = 0; i < n; i++)
+            for (uint32_t g = 0; g < 4; g++) {
+                if (reads_outside<SINTER_Q4_K>(n, i, g)) printf("q4_k %u of %u group %u\n", i, n, g);
+                if (reads_outside<SINTER_Q6_K>(n, i, g)) printf("q6_k %u of %u group %u\n", i, n, g);
+            }
+    return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def host_prog(sn, tmp_path_factory):
+    import build
+    d = tmp_path_factory.mktemp("ubatch_host")
+    (d / "t.hip").write_text(SRC)
+    exe = d / "t"
+    subprocess.run([build.hipcc(), "--offload-arch=gfx950", "--offload-host-only", "-O1", "-std=c++17",
+                    "-I", os.path.join(PKG, "csrc"), "-I", os.path.join(ROOT, "include"), str(d / "t.hip"), "-o", str(exe),
+                    "-L", PKG, "-lsinter", "-Wl,-rpath," + PKG, "-Wl,--unresolved-symbols=ignore-all"],
+                   check=True, capture_output=True)
+    return str(exe)
+
+
+def test_weight_loads_stay_in_the_operand(host_prog):
+    """Matrices of 1 to 8 blocks (an odd number of 210-byte Q6_K blocks ends
+    between 4-byte boundaries): no loaded register holds a byte outside."""
+    assert subprocess.run([host_prog], check=True, capture_output=True, text=True).stdout == ""
