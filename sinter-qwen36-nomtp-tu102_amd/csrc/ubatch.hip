@@ -679,12 +679,11 @@ __global__ __launch_bounds__(256) void conv_silu_kernel(const float *__restrict_
 // four partial sums (element i into sum i / 4) over its chunks g + 32,
 // g + 48, ... and then g and g + 16; the row adds them as
 // (s0 + s1) + (s2 + s3) and by its DPP butterfly, the wave its four rows in
-// order, the workgroup its four waves in order.  Those are the first four
-// waves; the normalised row is quantised by up to 16, wave v blocks v,
-// v + 16, ..., the first two of them loaded before the sum: a token is one
-// chain of latencies (four waves with each block's load behind the sum: 9.1
-// us at K 5120, 24 tokens, 5.0 us so).
-constexpr uint32_t UB_NORM_WAVES = 16;
+// order, the workgroup its four waves in order.  Those are the first four of NW
+// waves; the normalised row is quantised by all, wave v blocks v, v + NW, ....
+// PRE: everything the sum reads, and the wave's first two blocks, are loaded
+// at once ahead of it (a row is one chain of latencies), for twice the
+// registers and loads past a short row's end.
 __device__ __forceinline__ void ub_add_sq(const float4 x[4], double s4[4]) {
 #pragma unroll
     for (uint32_t q = 0; q < 4; q++) {
@@ -694,9 +693,10 @@ __device__ __forceinline__ void ub_add_sq(const float4 x[4], double s4[4]) {
         s4[q] += (double)(x[q].w * x[q].w);
     }
 }
-__global__ __launch_bounds__(64 * UB_NORM_WAVES) void rmsnorm_quant_q8k_kernel(const float *__restrict__ x,
-                                                                              const float *__restrict__ w, float eps,
-                                                                              uint32_t k, uint8_t *__restrict__ xq) {
+template <uint32_t NW, bool PRE>
+__global__ __launch_bounds__(64 * NW) void rmsnorm_quant_q8k_kernel(const float *__restrict__ x,
+                                                                   const float *__restrict__ w, float eps, uint32_t k,
+                                                                   uint8_t *__restrict__ xq) {
     __shared__ double red[4];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, r = tid & 15u, g = tid >> 4, nchunk = k / 256u;
     const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -706,15 +706,17 @@ __global__ __launch_bounds__(64 * UB_NORM_WAVES) void rmsnorm_quant_q8k_kernel(c
         for (uint32_t q = 0; q < 4; q++) v[q] = ((const float4 *)(xr + 256u * min(c, nchunk - 1u) + 16u * r))[q];
     };
     float4 a[4], b[4], xv[2], gv[2];
-    if (wv < 4u) {
-        chunk(g, a);
-        chunk(g + 16u, b);
-    }
+    if constexpr (PRE) {
+        if (wv < 4u) {
+            chunk(g, a);
+            chunk(g + 16u, b);
+        }
 #pragma unroll
-    for (uint32_t j = 0; j < 2; j++) {
-        const uint32_t bl = min(wv + UB_NORM_WAVES * j, nchunk - 1u);
-        xv[j] = ((const float4 *)(xr + 256u * bl))[lane];
-        gv[j] = w ? ((const float4 *)(w + 256u * bl))[lane] : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+        for (uint32_t j = 0; j < 2; j++) {
+            const uint32_t bl = min(wv + NW * j, nchunk - 1u);
+            xv[j] = ((const float4 *)(xr + 256u * bl))[lane];
+            gv[j] = w ? ((const float4 *)(w + 256u * bl))[lane] : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+        }
     }
     if (wv < 4u) {
         double s4[4] = {0.0, 0.0, 0.0, 0.0};
@@ -723,8 +725,14 @@ __global__ __launch_bounds__(64 * UB_NORM_WAVES) void rmsnorm_quant_q8k_kernel(c
             chunk(c, v);
             ub_add_sq(v, s4);
         }
-        if (g < nchunk) ub_add_sq(a, s4);
-        if (g + 16u < nchunk) ub_add_sq(b, s4);
+        if (g < nchunk) {
+            if constexpr (!PRE) chunk(g, a);
+            ub_add_sq(a, s4);
+        }
+        if (g + 16u < nchunk) {
+            if constexpr (!PRE) chunk(g + 16u, b);
+            ub_add_sq(b, s4);
+        }
         double s = row16_sum_f64((s4[0] + s4[1]) + (s4[2] + s4[3]));
         s = ((readlane_f64(s, 0) + readlane_f64(s, 16)) + readlane_f64(s, 32)) + readlane_f64(s, 48);
         if (lane == 0) red[wv] = s;
@@ -739,10 +747,12 @@ __global__ __launch_bounds__(64 * UB_NORM_WAVES) void rmsnorm_quant_q8k_kernel(c
         if (w) { e[0] = e[0] * gm.x; e[1] = e[1] * gm.y; e[2] = e[2] * gm.z; e[3] = e[3] * gm.w; }
         quant_block_q8k(e, lane, orow + (size_t)bl * Q8K_BYTES);
     };
+    if constexpr (PRE) {
 #pragma unroll
-    for (uint32_t j = 0; j < 2; j++)
-        if (wv + UB_NORM_WAVES * j < nchunk) quant(wv + UB_NORM_WAVES * j, xv[j], gv[j]);
-    for (uint32_t bl = wv + 2u * UB_NORM_WAVES; bl < nchunk; bl += UB_NORM_WAVES) {
+        for (uint32_t j = 0; j < 2; j++)
+            if (wv + NW * j < nchunk) quant(wv + NW * j, xv[j], gv[j]);
+    }
+    for (uint32_t bl = wv + (PRE ? 2u * NW : 0u); bl < nchunk; bl += NW) {
         const float4 v = ((const float4 *)(xr + 256u * bl))[lane];
         quant(bl, v, w ? ((const float4 *)(w + 256u * bl))[lane] : v);
     }
@@ -909,8 +919,22 @@ extern "C" int sinter_rmsnorm_quant_q8k_ubatch(const float *x, const float *w, f
     if ((uintptr_t)x % 16u || (uintptr_t)w % 16u || (uintptr_t)xq % 4u)
         return set_error(SINTER_ERR_ARG, "rmsnorm_quant_q8k_ubatch: alignment (x, w 16 bytes, xq 4 bytes)");
     if (!(eps >= 0.0f)) return set_error(SINTER_ERR_ARG, "rmsnorm_quant_q8k_ubatch: eps must be >= 0");
-    hipLaunchKernelGGL(rmsnorm_quant_q8k_kernel, dim3(n_tokens), dim3(64 * UB_NORM_WAVES), 0, (hipStream_t)stream, x, w, eps,
-                       (uint32_t)k, (uint8_t *)xq);
+    auto launch = [&](auto kernel, uint32_t waves) {
+        hipLaunchKernelGGL(kernel, dim3(n_tokens), dim3(64 * waves), 0, (hipStream_t)stream, x, w, eps, (uint32_t)k,
+                           (uint8_t *)xq);
+    };
+    // Up to one row per CU a row's latency is the time: 16 waves (us, four
+    // waves with their loads behind the sum -> so: K 5120, 24 rows 7.3 -> 3.5,
+    // 17408 20.0 -> 7.2).  Then 8, while a CU's rows are few for their length
+    // (5120, 512 rows 8.0, 16 waves 6.3, 8 waves 5.1).  Past that the waves
+    // that start and the registers they hold are the time: 4 without PRE
+    // (1024, 65536 rows: 16 waves 512, 4 with PRE 169, without 106; 5120, 8192
+    // rows: 84, 55, 49; 2048, 768 rows: 8 waves 4.7, 1024 rows: 5.7, 4 without
+    // PRE 4.7).
+    const uint32_t nchunk = (uint32_t)(k / 256);
+    if (n_tokens <= 256) launch(rmsnorm_quant_q8k_kernel<16, true>, 16);
+    else if (nchunk >= 8 && n_tokens <= 96ull * nchunk) launch(rmsnorm_quant_q8k_kernel<8, true>, 8);
+    else launch(rmsnorm_quant_q8k_kernel<4, false>, 4);
     return hip_ok(hipGetLastError(), "rmsnorm_quant_q8k_ubatch: launch") ? SINTER_OK : SINTER_ERR_HIP;
 }
 

@@ -352,3 +352,29 @@ def test_conv_silu_ubatch_token_edges(sn, orc, torch_gpu, dconv, n_tok):
     """Ubatches shorter than the conv's history (old state entries move up) and
     around a thread's eight tokens, for every tap count, channels off 256."""
     test_conv_silu_ubatch_matches_oracle_token_loop(sn, orc, torch_gpu, 300, dconv, n_tok)
+
+
+@pytest.mark.parametrize("k,n_tok", [(2048, 256), (2048, 257), (2048, 768), (2048, 769), (1792, 257), (8448, 300)])
+def test_rmsnorm_quant_q8k_ubatch_wave_rule(sn, orc, torch_gpu, k, n_tok):
+    """Both sides of the launch's lines: 16 waves a row up to 256 rows, 8 from
+    8 blocks a row up to 96 rows per block, 4 past that."""
+    test_rmsnorm_quant_q8k_ubatch_matches_oracle(sn, orc, torch_gpu, k, n_tok, True)
+
+
+def test_rmsnorm_quant_q8k_ubatch_many_rows(sn, torch_gpu):
+    """2^22 rows (a launch holds fewer than 2^32 threads): 1024 times the same
+    4096 rows, each time the bytes that these rows alone give."""
+    torch, k, n, rep = torch_gpu, 256, 4096, 1024
+    x = torch.randn(n, k, device="cuda")
+    w = torch.rand(k, device="cuda") + 0.5
+    big = x.repeat(rep, 1)
+    one = torch.zeros(n * 292, dtype=torch.uint8, device="cuda")
+    many = torch.zeros(rep, n * 292, dtype=torch.uint8, device="cuda")
+    s = C.c_void_p(stream(torch))
+    torch.cuda.synchronize()
+    for t, src, dst in ((n, x, one), (n * rep, big, many)):
+        print(f"rmsnorm_quant_q8k_ubatch k={k} tokens={t}", flush=True)
+        sn.check(sn.lib().sinter_rmsnorm_quant_q8k_ubatch(C.c_void_p(src.data_ptr()), C.c_void_p(w.data_ptr()), 1e-6, k,
+                                                          t, C.c_void_p(dst.data_ptr()), s), "rmsnorm_quant")
+    torch.cuda.synchronize()
+    assert bool((many == one).all())
