@@ -7,7 +7,7 @@ oracle's (oracle/oracle.c or_block_term / or_gemv_q), and the single-token
 device GEMV is bit-exact against the same oracle (test_gpu_ops.py).
 
 Shapes cover one token, token counts that are not a multiple of the 16-token
-tile or of the 64-token weight pass, row counts that are not a multiple of
+tile or of a workgroup's tiles (up to 8), row counts that are not a multiple of
 the 16-row tile, odd block counts per row (Q6_K's 210-byte blocks then start
 on both 4-byte phases), K up to 17408, zero activations and activations over
 six decades of scale.  A second test fills the weight blocks with random
@@ -68,14 +68,11 @@ def test_gemv_ubatch_matches_per_token_gemv(sn, orc, torch_gpu, t, rows, k, n_to
 
 
 @pytest.mark.parametrize("t,rows,k,n_tok", [
-    (Q4_K, 16384, 512, 100),    # 256 row tiles: four token tiles per workgroup, the last group three
-    (Q4_K, 8192, 512, 64),      # 128 row tiles: two token tiles per workgroup
-    (Q6_K, 16384, 512, 100),
-    (Q6_K, 8192, 768, 40)])     # two token tiles per workgroup, the last group one
+    (Q4_K, 16384, 512, 100), (Q4_K, 8192, 512, 64), (Q6_K, 16384, 512, 100), (Q6_K, 8192, 768, 40)])
 def test_gemv_ubatch_multi_tile_workgroups(sn, orc, torch_gpu, t, rows, k, n_tok):
     """Shapes with enough row tiles that a workgroup takes several 16-token
-    tiles (its waves staging tiles 1-3, a partial last token group): the
-    production shapes of a batched prefill run this path."""
+    tiles, a partial last one among them, as the production shapes of a batched
+    prefill do."""
     w = synth_w(sn, t, rows, k, 700 + t + k + rows)
     xs = activations(k, n_tok, 2000 + rows)
     got = run_ubatch(sn, orc, torch_gpu, t, w, rows, k, xs)
@@ -83,17 +80,21 @@ def test_gemv_ubatch_multi_tile_workgroups(sn, orc, torch_gpu, t, rows, k, n_tok
         assert np.array_equal(got[j], orc.gemv(t, w, rows, k, x)), j
 
 
-@pytest.mark.parametrize("t,rows,k,n_tok", [
-    # one case for each compiled split of the launch (token tiles of 16 per
-    # workgroup; few- or many-token kernel), ragged rows and token tails, odd
-    # and even item counts
-    (Q4_K, 41, 1280, 1), (Q4_K, 17, 256, 19),                       # few-token, 1 tile (items % waves != 0)
-    (Q4_K, 8100, 768, 17), (Q4_K, 12289, 512, 20),                  # many-token, 1 and 2 tiles
-    (Q4_K, 12289, 768, 33), (Q4_K, 12289, 512, 63),                 # 3 and 4
-    (Q4_K, 4100, 768, 250), (Q4_K, 8100, 256, 201),                 # 6 and 8
-    (Q6_K, 41, 1280, 1), (Q6_K, 1000, 768, 129),                    # few-token, 1 and 2
-    (Q6_K, 12289, 768, 17), (Q6_K, 12289, 512, 33),                 # many-token, 2 and 3
-    (Q6_K, 3001, 768, 250), (Q6_K, 12289, 512, 65), (Q6_K, 8100, 768, 201)])   # 4, 6 and 8
+# Cases for each compiled split of the launch (the kernel, and its 16-token
+# tiles per workgroup): ragged rows and token tails, odd and even item counts.
+# test_ubatch_host.py holds each to the split named beside it.
+EVERY_SPLIT = [
+    (Q4_K, 41, 1280, 1, "few", 1), (Q4_K, 17, 256, 19, "few", 1),   # (items % waves != 0)
+    (Q4_K, 8100, 768, 17, "many", 1), (Q4_K, 12289, 512, 20, "many", 2),
+    (Q4_K, 12289, 768, 33, "many", 3), (Q4_K, 12289, 512, 63, "many", 4),
+    (Q4_K, 4100, 768, 250, "many", 6), (Q4_K, 8100, 256, 201, "many", 8),
+    (Q6_K, 41, 1280, 1, "few", 1), (Q6_K, 1000, 768, 129, "few", 1),
+    (Q6_K, 5120, 768, 24, "few", 2), (Q6_K, 1500, 1280, 130, "few", 2),
+    (Q6_K, 12289, 768, 17, "many", 2), (Q6_K, 12289, 512, 33, "many", 3),
+    (Q6_K, 3001, 768, 250, "many", 4), (Q6_K, 12289, 512, 65, "many", 6), (Q6_K, 8100, 768, 201, "many", 8)]
+
+
+@pytest.mark.parametrize("t,rows,k,n_tok", [c[:4] for c in EVERY_SPLIT])
 def test_gemv_ubatch_every_split(sn, orc, torch_gpu, t, rows, k, n_tok):
     """Exact sums and the declared fold order: bit-identical on every split."""
     w = synth_w(sn, t, rows, k, 900 + t + k + rows)

@@ -1,9 +1,13 @@
 """The host-computable parts of the batched GEMV (csrc/ubatch.hip), compiled
-for the CPU: which bytes a weight item's loads depend on (no GPU)."""
+for the CPU: which bytes a weight item's loads depend on, and the split that a
+launch takes (no GPU)."""
 import os
+import re
 import subprocess
 
 import pytest
+
+from test_gpu_ubatch import EVERY_SPLIT
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PKG = os.path.join(ROOT, "sinter-qwen36-nomtp-tu102_amd")
@@ -32,7 +36,24 @@ static bool reads_outside(uint32_t n, uint32_t i, uint32_t g) {
     return memcmp(item[0], item[1], sizeof(Item)) != 0;
 }
 
-int main() {
+template <int WT>
+static void split(long rows, long k, long n_tok) {
+    UbArgs a = {};
+    a.nb = (uint32_t)(k / 256);
+    a.n_tok = (uint32_t)n_tok;
+    a.n_seg = 1;
+    a.rows[0] = (uint32_t)rows;
+    const UbSplit p = ub_split<WT>(a);
+    printf("%s %u %llu\n", p.few ? "few" : "many", p.nt, (unsigned long long)p.wgs);
+}
+
+int main(int argc, char **argv) {
+    if (argc > 1) {   // TYPE ROWS K TOKENS ...
+        for (int i = 1; i + 3 < argc; i += 4)
+            (atoi(argv[i]) == SINTER_Q4_K ? split<SINTER_Q4_K> : split<SINTER_Q6_K>)(atol(argv[i + 1]), atol(argv[i + 2]),
+                                                                                     atol(argv[i + 3]));
+        return 0;
+    }
     for (uint32_t n = 1; n <= 8; n++)
         for (uint32_t i = 0; i < n; i++)
             for (uint32_t g = 0; g < 4; g++) {
@@ -61,3 +82,22 @@ def test_weight_loads_stay_in_the_operand(host_prog):
     """Matrices of 1 to 8 blocks (an odd number of 210-byte Q6_K blocks ends
     between 4-byte boundaries): no loaded register holds a byte outside."""
     assert subprocess.run([host_prog], check=True, capture_output=True, text=True).stdout == ""
+
+
+def splits(host_prog, cases):
+    """[(kernel, token tiles per workgroup, workgroups)] of (type, rows, k, tokens)."""
+    args = [str(v) for c in cases for v in c[:4]]
+    out = subprocess.run([host_prog, *args], check=True, capture_output=True, text=True).stdout.splitlines()
+    return [(f[0], int(f[1]), int(f[2])) for f in map(str.split, out)]
+
+
+def test_every_split_case_takes_the_split_it_names(host_prog):
+    """The GPU test of every compiled split reaches each of them, whatever the
+    prices that choose are fitted to next."""
+    got = splits(host_prog, EVERY_SPLIT)
+    assert [g[:2] for g in got] == [c[4:] for c in EVERY_SPLIT]
+    src = open(os.path.join(PKG, "csrc", "ubatch.hip")).read()
+    launch = src[src.index("hipError_t launch_ubatch("):src.index("hipError_t launch_gemv_ubatch(")]
+    compiled = {(k, int(nt)) for f, k in (("launch_gemv", "few"), ("launch_gemm", "many"))
+                for nt in re.findall(f + r"<WT, (\d+)>", launch)}
+    assert compiled == {c[4:] for c in EVERY_SPLIT}
