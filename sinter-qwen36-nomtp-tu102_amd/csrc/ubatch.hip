@@ -270,6 +270,13 @@ __device__ __forceinline__ void ub_tile(const UbArgs &a, uint32_t &rt, uint32_t 
 // bytes; chunk c of token r lies in slot c ^ (r % 16), so the 16 tokens' reads
 // of one chunk fall on distinct banks without padding, which the DMA's
 // contiguous kilobyte per wave could not leave.
+//
+// SHORT: rows of at most UB_SHORT items.  Both buffers are filled and both
+// items' weights loaded before the first is multiplied, and nothing is loaded
+// ahead, so a workgroup reads each byte once and a CU holds twice the
+// workgroups (the loop below loads past the row's end: its items again, never
+// used).  us, the loop or the few-token kernel -> so: Q6_K 40000 x 512, 1 token
+// 9.8 -> 6.4, 256 tokens 26.5 -> 25.0; Q4_K 40000 x 256, 64 tokens 8.3 -> 6.3.
 constexpr uint32_t UB_THREADS = 256;
 constexpr uint32_t UB_WG_ROWS = UB_ROWS * (UB_THREADS / 64u);
 constexpr uint32_t UB_TILE_BYTES = UB_TOK * 256u;
@@ -278,9 +285,10 @@ template <uint32_t NT>
 constexpr uint32_t ub_buf() { return NT * (UB_TILE_BYTES + UB_TOK * 8u); }
 // the DMA's 32-bit lane offsets reach 128 tokens of items
 constexpr uint32_t UB_MAX_NB = 50000;
+constexpr uint32_t UB_SHORT = 2;
 
-template <int WT, uint32_t NT>
-__global__ __launch_bounds__(UB_THREADS, 2) void ubatch_gemm_kernel(UbArgs a) {
+template <int WT, uint32_t NT, bool SHORT>
+__global__ __launch_bounds__(UB_THREADS, SHORT ? 4 : 2) void ubatch_gemm_kernel(UbArgs a) {
     __shared__ __attribute__((aligned(16))) unsigned char xs[2 * ub_buf<NT>()];
     LDS unsigned char *L = (LDS unsigned char *)xs;
     const uint32_t lbase = (uint32_t)(uintptr_t)L;
@@ -314,32 +322,33 @@ __global__ __launch_bounds__(UB_THREADS, 2) void ubatch_gemm_kernel(UbArgs a) {
 #pragma unroll
         for (uint32_t v = 0; v < 4; v++) acc[t][v] = 0.0;
 
-    float dxn = 0.0f;
+    // item i's codes into buffer buf; its d of the thread's token
     auto stage = [&](uint32_t i, uint32_t buf) {
         const uint8_t *q = xp + (size_t)i * Q8K_BYTES;
         const uintptr_t p = (uintptr_t)q;
 #pragma unroll
         for (uint32_t j = 0; j < NT; j++)
             lds_dma16<false>(p, xo[j], lbase + buf * ub_buf<NT>() + j * UB_TILE_BYTES + wv * 1024u);
-        dxn = *(const float *)(q + dxo);
+        return *(const float *)(q + dxo);
     };
-    auto park = [&](uint32_t buf) {
+    auto park = [&](uint32_t buf, float dxn) {
         if (threadIdx.x < UB_TOK * NT)
             *reinterpret_cast<LDS double *>(L + buf * ub_buf<NT>() + NT * UB_TILE_BYTES + 8u * threadIdx.x) = (double)dxn;
     };
     struct AFrag { v4i x[4]; v2d d0, d1; };
+    auto read = [&](uint32_t buf, uint32_t t) {   // tile t of buffer buf
+        const LDS unsigned char *xb = L + buf * ub_buf<NT>(), *dxs = xb + NT * UB_TILE_BYTES + 32u * g;
+        AFrag f;
+#pragma unroll
+        for (uint32_t m = 0; m < 4; m++) f.x[m] = *reinterpret_cast<const LDS v4i *>(xb + ao[m] + t * UB_TILE_BYTES);
+        const LDS v2d *q = reinterpret_cast<const LDS v2d *>(dxs + t * UB_TOK * 8u);
+        f.d0 = q[0];
+        f.d1 = q[1];
+        return f;
+    };
     // item i: its codes in buffer `buf`, its weights in w
     auto item = [&](uint32_t i, uint32_t buf, WItem<WT> &w) {
-        const LDS unsigned char *xb = L + buf * ub_buf<NT>(), *dxs = xb + NT * UB_TILE_BYTES + 32u * g;
-        auto lda = [&](uint32_t t) {
-            AFrag f;
-#pragma unroll
-            for (uint32_t m = 0; m < 4; m++) f.x[m] = *reinterpret_cast<const LDS v4i *>(xb + ao[m] + t * UB_TILE_BYTES);
-            const LDS v2d *q = reinterpret_cast<const LDS v2d *>(dxs + t * UB_TOK * 8u);
-            f.d0 = q[0];
-            f.d1 = q[1];
-            return f;
-        };
+        auto lda = [&](uint32_t t) { return read(buf, t); };
         // (the empty asm statements keep the compiler from sinking the
         // arithmetic past the loads that it is to run beside, or past the
         // barrier: the unpacking would wait for the loads behind it)
@@ -354,7 +363,7 @@ __global__ __launch_bounds__(UB_THREADS, 2) void ubatch_gemm_kernel(UbArgs a) {
         // the next item's activations, then the weights of the one after it:
         // loads complete in order, so the wait below leaves the weights in
         // flight (past the end: the last item again, never used)
-        stage(min(i + 1u, nb - 1u), buf ^ 1u);
+        float dxn = stage(min(i + 1u, nb - 1u), buf ^ 1u);
         sched_fence();
         w.load(wp + (size_t)min(i + 2u, nb - 1u) * WItem<WT>::BYTES, g);
         AFrag f = lda(0), fn;
@@ -387,22 +396,51 @@ __global__ __launch_bounds__(UB_THREADS, 2) void ubatch_gemm_kernel(UbArgs a) {
         // DMAs: loads complete in order, so they have landed (the weights
         // behind them may still fly)
         asm volatile("" : "+v"(dxn)::"memory");
-        park(buf ^ 1u);
+        park(buf ^ 1u, dxn);
         __syncthreads();
     };
+    // the same item with nothing loaded beside it
+    auto item_only = [&](uint32_t buf, const WItem<WT> &w) {
+        BItem b;
+        w.unpack(b, g);
+#pragma unroll
+        for (uint32_t t = 0; t < NT; t++) {
+            const AFrag f = read(buf, t);
+            const double dx[4] = {f.d0[0], f.d0[1], f.d1[0], f.d1[1]};
+            double tm[4];
+            tile_terms<WT>(tile_sums<WT>(f.x, b), (double)b.dw, (double)b.dmin, dx, tm);
+#pragma unroll
+            for (uint32_t v = 0; v < 4; v++) acc[t][v] += tm[v];
+        }
+    };
     WItem<WT> w0, w1;
-    stage(0, 0);
-    sched_fence();
-    w0.load(wp, g);
-    w1.load(wp + (size_t)min(1u, nb - 1u) * WItem<WT>::BYTES, g);
-    park(0);
-    dma_wait();
-    __syncthreads();
-    for (uint32_t i = 0; i < nb; i += 2) {
-        item(i, 0, w0);
-        if (i + 1u < nb) item(i + 1u, 1, w1);
+    if constexpr (SHORT) {
+        w0.load(wp, g);
+        const float d0 = stage(0, 0);
+        if (nb > 1u) {
+            w1.load(wp + WItem<WT>::BYTES, g);
+            const float d1 = stage(1, 1);
+            park(1, d1);
+        }
+        park(0, d0);
+        dma_wait();
+        __syncthreads();
+        item_only(0, w0);
+        if (nb > 1u) item_only(1, w1);
+    } else {
+        const float d0 = stage(0, 0);
+        sched_fence();
+        w0.load(wp, g);
+        w1.load(wp + (size_t)min(1u, nb - 1u) * WItem<WT>::BYTES, g);
+        park(0, d0);
+        dma_wait();
+        __syncthreads();
+        for (uint32_t i = 0; i < nb; i += 2) {
+            item(i, 0, w0);
+            if (i + 1u < nb) item(i + 1u, 1, w1);
+        }
+        dma_wait();   // (the last item's staging must not outlive the workgroup's LDS)
     }
-    dma_wait();   // (the last item's staging must not outlive the workgroup's LDS)
 
     if (row < rows) {
         float *y = a.y[sg] + row;
@@ -766,12 +804,20 @@ using namespace sinter;
 namespace sinter {
 namespace {
 
-// The split of a launch: token tiles per workgroup, few-token or many-token kernel.
+// The split of a launch: the kernel and its token tiles per workgroup.
 struct UbSplit {
-    bool few;
+    enum Kernel { FEW, MANY, SHORT } kernel;
     uint32_t nt, wg_rows, n_tg;
     uint64_t wgs;
 };
+template <int WT>
+UbSplit ub_split_of(const UbArgs &a, UbSplit::Kernel kernel, uint32_t nt) {
+    UbSplit s = {kernel, nt, kernel == UbSplit::FEW ? UB_ROWS : UB_WG_ROWS, 0, 0};
+    s.n_tg = ((a.n_tok + UB_TOK - 1) / UB_TOK + nt - 1) / nt;
+    for (uint32_t i = 0; i < a.n_seg; i++) s.wgs += ((uint64_t)a.rows[i] + s.wg_rows - 1) / s.wg_rows;
+    s.wgs *= s.n_tg;
+    return s;
+}
 
 // The cheapest of the compiled splits by a cost per item, fitted to times of
 // 11 matrices (32..34816 rows, K 4096..17408) x 10 token counts (8..512); ns:
@@ -784,41 +830,52 @@ struct UbSplit {
 // 8 143; at 5 tokens few-token 37, many-token 90; 151936 x 5120 at 1, 5 and 16
 // tokens: few-token 154, 162, 193, many-token 175, 186, 195.  Q4_K 34816 x 5120 at 256:
 // nt 2 205, 4 180, 6 181, 8 166; 8192 x 5120 at 24: few-token 15, nt 1 15.5.
+// Short rows are mostly start-up, which these prices leave out: one item goes
+// to SHORT, two do where the few-token kernel would take them with more than
+// two workgroups per CU, or the many-token kernel with many or for one or two
+// token tiles (us, the price's choice -> SHORT: Q6_K 160000 x 256, 1 token 30.1
+// -> 8.5, 10000 x 256, 16 tokens 4.9 -> 3.4, 40000 x 512, 16 tokens 9.9 -> 6.9,
+// 20 tokens 10.1 -> 7.8; but 1000 x 512, 64 tokens 3.7, SHORT 4.3, and 5000 x
+// 512, 256 tokens 7.6, SHORT 8.0).  The more workgroups one token tile each
+// would give, the more tiles one takes (us at nt 1, 2, 4: Q4_K 20000 x 256, 64
+// tokens 4.8, 5.7, 5.4, 40000 x 256, 64 tokens 7.2, 6.3, 6.7, 160000 x 256, 40
+// tokens 15.7, 15.6, 13.6; Q6_K 10000 x 256, 64 tokens 4.6, 4.5, 5.0, 40000 x
+// 256, 64 tokens 9.7, 7.3, 7.1).
 template <int WT>
 UbSplit ub_split(const UbArgs &a) {
     constexpr bool Q4 = WT == SINTER_Q4_K;
     const uint32_t tiles = (a.n_tok + UB_TOK - 1) / UB_TOK;
     UbSplit best = {};
     double cost = 1e300;
-    auto consider = [&](bool few, uint32_t nt, double lone, double thr, double start) {
-        UbSplit s;
-        s.few = few;
-        s.nt = nt;
-        s.wg_rows = few ? UB_ROWS : UB_WG_ROWS;
-        s.n_tg = (tiles + nt - 1) / nt;
-        uint64_t n_rt = 0;
-        for (uint32_t i = 0; i < a.n_seg; i++) n_rt += ((uint64_t)a.rows[i] + s.wg_rows - 1) / s.wg_rows;
-        s.wgs = n_rt * s.n_tg;
+    auto consider = [&](UbSplit::Kernel kernel, uint32_t nt, double lone, double thr, double start) {
+        const UbSplit s = ub_split_of<WT>(a, kernel, nt);
         const double w = (double)s.wgs / 256.0;
         double c;
-        if (few) c = std::max(lone, start + w * thr);
+        if (kernel == UbSplit::FEW) c = std::max(lone, start + w * thr);
         else c = start + (w <= 1.0 ? lone : std::max(lone, std::floor(w) * thr) + (w > std::floor(w) ? 0.65 * thr : 0.0));
         if (c < cost) { cost = c; best = s; }
     };
     // (not compiled, as never the cheapest: few-token nt 2 for Q4_K, whose
     // unpacking is cheap enough to repeat; many-token nt 1 for Q6_K, whose is not)
     const uint32_t tok = std::min(a.n_tok, UB_TOK);
-    consider(true, 1, Q4 ? 370 : 560, Q4 ? 166 : 200 + 3 * tok, Q4 ? 200 : 150);
-    if (!Q4 && tiles > 1) consider(true, 2, 700, 420, 150);
+    consider(UbSplit::FEW, 1, Q4 ? 370 : 560, Q4 ? 166 : 200 + 3 * tok, Q4 ? 200 : 150);
+    if (!Q4 && tiles > 1) consider(UbSplit::FEW, 2, 700, 420, 150);
     if (a.nb > UB_MAX_NB) return best;
     for (uint32_t nt : {Q4 ? 1u : 2u, 2u, 3u, 4u, 6u, 8u})
-        consider(false, nt, Q4 ? 477 + 168 * nt : 1030 + 108 * nt, Q4 ? 190 + 215 * nt : 550 + 150 * nt, 125);
+        consider(UbSplit::MANY, nt, Q4 ? 477 + 168 * nt : 1030 + 108 * nt, Q4 ? 190 + 215 * nt : 550 + 150 * nt, 125);
+    if (a.nb <= UB_SHORT) {
+        const uint64_t w = ub_split_of<WT>(a, UbSplit::SHORT, 1).wgs, few = ub_split_of<WT>(a, UbSplit::FEW, 1).wgs;
+        if (a.nb == 1 || (best.kernel == UbSplit::FEW ? few > 512 : w >= 1400 || tiles <= 2))
+            return ub_split_of<WT>(a, UbSplit::SHORT, w >= (Q4 ? 4096 : 1024) && tiles > 2  ? 4
+                                                      : w >= (Q4 ? 1400 : 512) && tiles > 1 ? 2
+                                                                                            : 1);
+    }
     return best;
 }
 
-template <int WT, uint32_t NT>
+template <int WT, uint32_t NT, bool SHORT = false>
 void launch_gemm(const UbArgs &a, uint32_t grid, hipStream_t s) {
-    hipLaunchKernelGGL((ubatch_gemm_kernel<WT, NT>), dim3(grid), dim3(UB_THREADS), 0, s, a);
+    hipLaunchKernelGGL((ubatch_gemm_kernel<WT, NT, SHORT>), dim3(grid), dim3(UB_THREADS), 0, s, a);
 }
 template <int WT, uint32_t NT>
 void launch_gemv(const UbArgs &a, uint32_t grid, hipStream_t s) {
@@ -836,7 +893,11 @@ hipError_t launch_ubatch(UbArgs &a, hipStream_t s) {
         n_rt += (uint32_t)(((uint64_t)a.rows[i] + p.wg_rows - 1) / p.wg_rows);
     }
     const uint32_t grid = (uint32_t)p.wgs;
-    if (p.few) {
+    if (p.kernel == UbSplit::SHORT) {
+        if (p.nt == 1) launch_gemm<WT, 1, true>(a, grid, s);
+        else if (p.nt == 2) launch_gemm<WT, 2, true>(a, grid, s);
+        else launch_gemm<WT, 4, true>(a, grid, s);
+    } else if (p.kernel == UbSplit::FEW) {
         if constexpr (WT == SINTER_Q6_K) {
             if (p.nt == 2) {
                 launch_gemv<WT, 2>(a, grid, s);

@@ -84,14 +84,18 @@ def test_gemv_ubatch_multi_tile_workgroups(sn, orc, torch_gpu, t, rows, k, n_tok
 # tiles per workgroup): ragged rows and token tails, odd and even item counts.
 # test_ubatch_host.py holds each to the split named beside it.
 EVERY_SPLIT = [
-    (Q4_K, 41, 1280, 1, "few", 1), (Q4_K, 17, 256, 19, "few", 1),   # (items % waves != 0)
-    (Q4_K, 8100, 768, 17, "many", 1), (Q4_K, 12289, 512, 20, "many", 2),
+    (Q4_K, 41, 1280, 1, "few", 1), (Q4_K, 17, 512, 19, "few", 1),   # (items % waves != 0)
+    (Q4_K, 8100, 768, 17, "many", 1), (Q4_K, 12289, 768, 20, "many", 2),
     (Q4_K, 12289, 768, 33, "many", 3), (Q4_K, 12289, 512, 63, "many", 4),
-    (Q4_K, 4100, 768, 250, "many", 6), (Q4_K, 8100, 256, 201, "many", 8),
+    (Q4_K, 4100, 768, 250, "many", 6), (Q4_K, 8100, 768, 201, "many", 8),
     (Q6_K, 41, 1280, 1, "few", 1), (Q6_K, 1000, 768, 129, "few", 1),
     (Q6_K, 5120, 768, 24, "few", 2), (Q6_K, 1500, 1280, 130, "few", 2),
     (Q6_K, 12289, 768, 17, "many", 2), (Q6_K, 12289, 512, 33, "many", 3),
-    (Q6_K, 3001, 768, 250, "many", 4), (Q6_K, 12289, 512, 65, "many", 6), (Q6_K, 8100, 768, 201, "many", 8)]
+    (Q6_K, 3001, 768, 250, "many", 4), (Q6_K, 12289, 512, 65, "many", 6), (Q6_K, 8100, 768, 201, "many", 8),
+    (Q4_K, 17, 256, 19, "short", 1), (Q4_K, 10001, 512, 16, "short", 1), (Q4_K, 8100, 256, 201, "short", 2),
+    (Q4_K, 20001, 512, 90, "short", 2), (Q4_K, 20001, 256, 219, "short", 4), (Q4_K, 20001, 512, 219, "short", 4),
+    (Q6_K, 17, 256, 19, "short", 1), (Q6_K, 10001, 512, 5, "short", 1), (Q6_K, 10001, 256, 57, "short", 2),
+    (Q6_K, 20001, 512, 19, "short", 2), (Q6_K, 10001, 256, 120, "short", 4), (Q6_K, 20001, 512, 82, "short", 4)]
 
 
 @pytest.mark.parametrize("t,rows,k,n_tok", [c[:4] for c in EVERY_SPLIT])

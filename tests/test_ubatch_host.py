@@ -44,7 +44,8 @@ static void split(long rows, long k, long n_tok) {
     a.n_seg = 1;
     a.rows[0] = (uint32_t)rows;
     const UbSplit p = ub_split<WT>(a);
-    printf("%s %u %llu\n", p.few ? "few" : "many", p.nt, (unsigned long long)p.wgs);
+    const char *kernel = p.kernel == UbSplit::FEW ? "few" : p.kernel == UbSplit::MANY ? "many" : "short";
+    printf("%s %u %llu\n", kernel, p.nt, (unsigned long long)p.wgs);
 }
 
 int main(int argc, char **argv) {
@@ -98,6 +99,7 @@ def test_every_split_case_takes_the_split_it_names(host_prog):
     assert [g[:2] for g in got] == [c[4:] for c in EVERY_SPLIT]
     src = open(os.path.join(PKG, "csrc", "ubatch.hip")).read()
     launch = src[src.index("hipError_t launch_ubatch("):src.index("hipError_t launch_gemv_ubatch(")]
-    compiled = {(k, int(nt)) for f, k in (("launch_gemv", "few"), ("launch_gemm", "many"))
-                for nt in re.findall(f + r"<WT, (\d+)>", launch)}
+    compiled = {(k, int(nt)) for f, k in (("launch_gemv<WT, {}>", "few"), ("launch_gemm<WT, {}>", "many"),
+                                          ("launch_gemm<WT, {}, true>", "short"))
+                for nt in re.findall(f.format(r"(\d+)"), launch)}
     assert compiled == {c[4:] for c in EVERY_SPLIT}
