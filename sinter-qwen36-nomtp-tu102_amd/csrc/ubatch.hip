@@ -853,6 +853,9 @@ UbSplit ub_split(const UbArgs &a) {
         double c;
         if (kernel == UbSplit::FEW) c = std::max(lone, start + w * thr);
         else c = start + (w <= 1.0 ? lone : std::max(lone, std::floor(w) * thr) + (w > std::floor(w) ? 0.65 * thr : 0.0));
+        // (a launch holds fewer than 2^32 threads; the few-token kernel's row
+        // tiles are the smaller: Q6_K with 1-4 tokens past 2^28 rows)
+        if (s.wgs > UINT32_MAX / UB_THREADS) c += 1e200;
         if (c < cost) { cost = c; best = s; }
     };
     // (not compiled, as never the cheapest: few-token nt 2 for Q4_K, whose

@@ -103,3 +103,16 @@ def test_every_split_case_takes_the_split_it_names(host_prog):
                                           ("launch_gemm<WT, {}, true>", "short"))
                 for nt in re.findall(f.format(r"(\d+)"), launch)}
     assert compiled == {c[4:] for c in EVERY_SPLIT}
+
+
+@pytest.mark.parametrize("t", [12, 14])
+def test_split_fits_a_launch_wherever_64_row_tiles_do(host_prog, t):
+    """A launch holds fewer than 2^32 threads (256 per workgroup): a matrix
+    that fits one with 64 rows and 64 tokens per workgroup is never split finer
+    than that allows, up to what 288 GB of weights hold."""
+    cases = [(t, rows, k, n) for k in (256, 512, 768, 1024, 5120) for n in (1, 2, 4, 5, 16, 17, 33, 64, 65, 129)
+             for rows in (2**22, 2**27, 2**28, 2**28 + 1, 300_000_000, 450_000_000, 2**30 - 64)
+             if rows * (k // 256) * (144 if t == 12 else 210) < 288e9 and -(-rows // 64) * -(-n // 64) * 256 < 2**32]
+    assert len(cases) > 100
+    for c, g in zip(cases, splits(host_prog, cases)):
+        assert g[2] * 256 < 2**32, (c, g)
