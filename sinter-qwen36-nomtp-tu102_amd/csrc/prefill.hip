@@ -377,7 +377,8 @@ static_assert(PF_Q8_VS + 32 * 8 * 4 <= PF_TILES, "Q8_0 tiles fit the tile region
 // queries' chunk-c rows in the decode attention's tiles; a row outside a
 // query's own range is masked out of its scores and enters its V sums as
 // fmaf(0, v, acc) (no change but the sign of a zero sum, which the Q8_K
-// quantisation of the attention output erases).  Per query the chunk partial
+// quantisation of the attention output erases), or not at all where v is not
+// finite.  Per query the chunk partial
 // -- the 8 row groups merged, O, M, L -- is the decode's, bit for bit.
 //
 // The decode's fmaf chains run on v_mfma_f32_16x16x1_4b_f32: four 16 x 16
@@ -398,7 +399,7 @@ static_assert(PF_Q8_VS + 32 * 8 * 4 <= PF_TILES, "Q8_0 tiles fit the tile region
 // tile's.  K rows lie in LDS as 16-byte chunks, chunk p at slot p ^ (row %
 // 16), so 16 rows' reads of one chunk hit distinct banks.  256 queries behind
 // 8192 positions, 27B shapes: 1.60 ms with VALU chains (8 queries per item),
-// 0.98 ms so.
+// 0.99 ms so.
 template <bool Q8>
 __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(AttnPrefill a, uint32_t cmax) {
     __shared__ __attribute__((aligned(16))) unsigned char tiles[PF_TILES];
@@ -571,7 +572,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(AttnPrefill 
                     vraw[i][gi] = *reinterpret_cast<const LDS u32x2 *>(vt + (2 * w + gi + 8 * i) * 512u + 8u * lane);
         }
         __syncthreads();
-        bool rescale;
+        bool changed;
+        const bool partial = my1 > my0 && (t0 < my0 || t0 + ATT_TILE > my1);
         {
             float sv[2], wg[2];
             bool ok[2];
@@ -604,18 +606,94 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(AttnPrefill 
             lrun = lc + ws;
             mrun = mn;
             if (hf == 0) CF[rr * PF_SLOTS + sq] = cf;
-            rescale = __builtin_amdgcn_ballot_w64(cf != 1.0f) != 0;
+            changed = cf != 1.0f;
         }
         // (weights and corrections are read back by this wave only: LDS
         // accesses of a wave complete in order)
-        if (rescale) {
+        if (__builtin_amdgcn_ballot_w64(changed || partial) != 0) {
+            if (__builtin_amdgcn_ballot_w64(changed) != 0) {
 #pragma unroll
-            for (uint32_t gi = 0; gi < 2; gi++) {
-                const f32x4 cv = *reinterpret_cast<const LDS f32x4 *>(CF + (2 * w + gi) * PF_SLOTS + 4 * lb);
+                for (uint32_t gi = 0; gi < 2; gi++) {
+                    const f32x4 cv = *reinterpret_cast<const LDS f32x4 *>(CF + (2 * w + gi) * PF_SLOTS + 4 * lb);
 #pragma unroll
-                for (uint32_t jj = 0; jj < 4; jj++)
+                    for (uint32_t jj = 0; jj < 4; jj++)
 #pragma unroll
-                    for (uint32_t e = 0; e < 16; e++) acc[gi][jj][e] = acc[gi][jj][e] * cv[e & 3u];
+                        for (uint32_t e = 0; e < 16; e++) acc[gi][jj][e] = acc[gi][jj][e] * cv[e & 3u];
+                }
+            }
+            // a tile with rows that some query does not hold: a V value in it
+            // that is not finite is added here, to the queries that hold its
+            // row, and is 0 below, where a zero weight would not keep it out of
+            // the others.  (Selects and no branches inside, and out of the
+            // loop's way: 256 queries behind 8192 positions 968 -> 985 us; a
+            // branch per value 989, behind 131008 10.90 and 11.21 ms.)
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(partial) != 0, 0)) {
+                // (the lane is opaque: addresses made of it would be kept in
+                // registers through the loop, and spill)
+                uint32_t ln = lane;
+                asm volatile("" : "+v"(ln));
+                const uint32_t n16 = ln & 15u, nb4 = ln >> 4;
+                LDS float *vs = reinterpret_cast<LDS float *>(Lu + PF_Q8_VS);
+                const uint32_t vo = (2 * w + ((ln >> 3) & 1u) + 8 * nb4) * 8 + (ln & 7u);   // the wave's 64 scales
+                bool bad = false;
+                if constexpr (Q8) {
+                    bad = !(fabsf(vs[vo]) < INFINITY);
+                } else {
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; i++)
+#pragma unroll
+                        for (uint32_t gi = 0; gi < 2; gi++) {
+                            const uint32_t x = ~vraw[i][gi].x & 0x7c007c00u, y = ~vraw[i][gi].y & 0x7c007c00u;
+                            bad |= !(x & 0xffffu) || !(x >> 16) || !(y & 0xffffu) || !(y >> 16);
+                        }
+                }
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad) != 0, 0)) {
+#pragma unroll 1
+                    for (uint32_t i = 0; i < 4; i++)
+#pragma unroll
+                        for (uint32_t gi = 0; gi < 2; gi++) {
+                            const uint32_t r = 2 * w + gi + 8 * i;
+                            // (query q's bounds: lane 2 q)
+                            const uint64_t holds = __builtin_amdgcn_ballot_w64(t0 + r >= my0 && t0 + r < my1) >> (8 * nb4);
+                            const f32x4 wq = *reinterpret_cast<const LDS f32x4 *>(W + r * PF_SLOTS + 4 * nb4);
+#pragma unroll
+                            for (uint32_t b4 = 0; b4 < 4; b4++) {
+                                sched_fence();
+                                float vd[4];
+                                if constexpr (!Q8) {
+                                    const u32x2 u = *reinterpret_cast<const LDS u32x2 *>(vt + r * 512u + 8u * (16 * b4 + n16));
+#pragma unroll
+                                    for (uint32_t k = 0; k < 4; k++) vd[k] = h2f((uint16_t)((k < 2 ? u.x : u.y) >> (16 * (k & 1u))));
+                                } else {
+                                    const uint32_t u = *reinterpret_cast<const LDS uint32_t *>(vt + r * 256u + 4u * (16 * b4 + n16));
+#pragma unroll
+                                    for (uint32_t k = 0; k < 4; k++)
+                                        vd[k] = (float)(int)(int8_t)((u >> (8 * k)) & 0xffu) * vs[r * 8 + ((16 * b4 + n16) >> 3)];
+                                }
+#pragma unroll
+                                for (uint32_t jj = 0; jj < 4; jj++)
+#pragma unroll
+                                    for (uint32_t v = 0; v < 4; v++) {
+                                        const float o = acc[gi][jj][4 * b4 + v], n = fmaf(wq[v], vd[jj], o);
+                                        acc[gi][jj][4 * b4 + v] = !(fabsf(vd[jj]) < INFINITY) && ((holds >> (2 * v)) & 1u) ? n : o;
+                                    }
+                            }
+                        }
+                    if constexpr (Q8) {
+                        if (bad) vs[vo] = 0.0f;
+                    } else {
+#pragma unroll
+                        for (uint32_t i = 0; i < 4; i++)
+#pragma unroll
+                            for (uint32_t gi = 0; gi < 2; gi++)
+#pragma unroll
+                                for (uint32_t k = 0; k < 2; k++) {
+                                    uint32_t &u = reinterpret_cast<uint32_t *>(&vraw[i][gi])[k];
+                                    if (!(~u & 0x7c00u)) u &= 0xffff0000u;
+                                    if (!(~u & 0x7c000000u)) u &= 0xffffu;
+                                }
+                    }
+                }
             }
         }
         float wt[4][2];
@@ -691,7 +769,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(AttnPrefill 
 #pragma unroll
             for (uint32_t dd = 0; dd < 8; dd++) o[dd] = fmaf(e, cv[dd], o[dd]);
         }
-        const uint32_t m0 = (uint32_t)__shfl((int)k0, (int)q, 64), m1 = (uint32_t)__shfl((int)k1, (int)q, 64);
+        const uint32_t m0 = (uint32_t)__shfl((int)my0, (int)(2 * q), 64), m1 = (uint32_t)__shfl((int)my1, (int)(2 * q), 64);
         if (m1 > m0) {
             const uint32_t PS = att_rec(HD);
             float *d = a.part + (((size_t)(q0 + q) * NQ + head) * C + c) * PS;

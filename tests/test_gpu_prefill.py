@@ -257,3 +257,57 @@ def test_batched_prefill_attention_query_blocks(sn, torch_gpu, kv, past, chunks,
     finally:
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("kv", ["f16", "q8_0"])
+@pytest.mark.parametrize("at", [0, 5, 15, 16, 30, 39])
+def test_batched_prefill_keeps_an_overflowing_value_to_its_rows(sn, torch_gpu, kv, at):
+    """A token whose values overflow the cache (an infinite f16, or Q8_0 block
+    scale) reaches only the queries that attend to it: the tokens before it in
+    the same blocks of queries are as one pass per token leaves them, and so
+    are those after it."""
+    cfg = small_config(sn, n_layer=2, n_ctx=64)
+    cfg.attn_every, cfg.t_kv = 1, sn.Q8_0 if kv == "q8_0" else sn.F16
+    rng = np.random.default_rng(7)
+    toks = [int(t) for t in rng.choice(cfg.n_vocab, 40, replace=False)]
+    SLOT_V = 7
+    a, b, probe = (sn.Model(cfg, seed=71) for _ in range(3))
+    try:
+        # each token's largest value in the first layer, where it depends on the token alone
+        probe.prefill(toks, 0, mode="tokenwise")
+        d, nb = probe.state(0, 1)
+        row = nb // cfg.n_ctx
+        rows = device_bytes(probe, d, nb).reshape(cfg.n_ctx, row)[:40]
+        if kv == "f16":
+            v = np.abs(rows.view(np.float16).astype(np.float32))
+        else:
+            v = rows.reshape(40, -1, 34)[:, :, :2].copy().view(np.float16).astype(np.float32)
+        big = v.reshape(40, -1).max(1)
+        order = np.argsort(big)
+        top, lim = order[-1], np.sqrt(big[order[-1]] * big[order[-2]])
+        toks[at], toks[top] = toks[top], toks[at]
+        # the value matrix scaled so that this token alone passes the f16 range
+        d, nb, t = a.tensor(0, SLOT_V)
+        w = device_bytes(a, d, nb).reshape(-1, sn.BLOCK_BYTES[t])
+        at_d = {sn.Q4_K: slice(0, 4), sn.Q6_K: slice(208, 210)}[t]
+        w[:, at_d] = (w[:, at_d].copy().view(np.float16).astype(np.float32) * (65520.0 / lim)).astype(np.float16).view(np.uint8)
+        for m in (a, b):
+            m.h2d(m.tensor(0, SLOT_V)[0], w.reshape(-1), nb)
+        print(f"overflowing value kv={kv} at {at} (largest {big[order[-1]]}, next {big[order[-2]]})", flush=True)
+        a.prefill(toks, 0, mode="batched")
+        b.prefill(toks, 0, mode="tokenwise")
+        for il in range(2):
+            for s in range(2):
+                da, n = a.state(il, s)
+                ga, gb = (device_bytes(m, m.state(il, s)[0], n).reshape(cfg.n_ctx, -1) for m in (a, b))
+                if kv == "f16":
+                    ga, gb = ga.view(np.float16), gb.view(np.float16)
+                    if (il, s) == (0, 1):
+                        assert np.isinf(ga).any(1).nonzero()[0].tolist() == [at]
+                    assert np.array_equal(ga, gb, equal_nan=True), (il, s)
+                else:
+                    assert np.array_equal(ga, gb), (il, s)
+        assert np.array_equal(a.logits(), b.logits(), equal_nan=True)
+    finally:
+        for m in (a, b, probe):
+            m.close()
