@@ -311,3 +311,42 @@ def test_batched_prefill_keeps_an_overflowing_value_to_its_rows(sn, torch_gpu, k
     finally:
         for m in (a, b, probe):
             m.close()
+
+
+def test_prefill_attention_keeps_subnormals(sn, orc, torch_gpu):
+    """The prefill attention's matrix instructions flush no subnormal: V sums of
+    weights around exp(-90) and values down to the smallest f16, in tiles whose
+    largest scores have V = 0, bit for bit the oracle's fmaf chains (the
+    launcher is internal to the library and found by its C++ name)."""
+    torch = torch_gpu
+    NQ, NKV, HD, T, pos0 = 8, 2, 256, 17, 190
+    rows = pos0 + T
+    rng = np.random.default_rng(5)
+    K = np.zeros((rows, NKV, HD), np.float16)
+    V = (rng.standard_normal((rows, NKV, HD)) * 10.0 ** rng.uniform(-7, 0, (rows, NKV, HD))).astype(np.float16)
+    high = np.arange(rows) // 8 % 4 == 0               # in every tile and row group
+    K[:, :, 0] = np.where(high[:, None], 0.0, rng.uniform(-103, -78, (rows, NKV)))
+    V[high] = 0
+    qr = np.zeros((T, NQ, HD), np.float32)
+    qr[:, :, 0] = rng.uniform(15.9, 16.1, (T, NQ))
+    qg = np.zeros((T, NQ, 2 * HD), np.float32)         # gate: sigmoid(0) = 1/2
+    dev = [torch.from_numpy(a).cuda() for a in (qr, qg, K.view(np.int16), V.view(np.int16))]
+    part = torch.zeros(T * NQ * 64 * (HD + 4), device="cuda")
+    out = torch.zeros(T, NQ, HD, device="cuda")
+    launch = sn.lib()["_ZN6sinter19launch_attn_prefillEPKfS1_PKvS3_jijjjjjjfPfS4_P12ihipStream_t"]
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    print("prefill attention of subnormal sums", flush=True)
+    u32 = C.c_uint32
+    assert launch(*(C.c_void_p(t.data_ptr()) for t in dev), u32(sn.F16), C.c_int32(pos0), u32(T), u32(NQ), u32(NKV), u32(HD),
+                  u32(64), u32(128), C.c_float(0.0625), C.c_void_p(part.data_ptr()), C.c_void_p(out.data_ptr()),
+                  C.c_void_p(s.cuda_stream)) == 0
+    torch.cuda.synchronize()
+    got, want = out.cpu().numpy(), np.zeros((T, NQ, HD), np.float32)
+    for t in range(T):
+        orc.lib().or_attn_split(qr[t].ctypes.data, K.ctypes.data, V.ctypes.data, orc.F16, pos0 + t + 1, NQ, NKV, HD, 0.0625,
+                                64, 128, want[t].ctypes.data)
+    want *= np.float32(0.5)
+    tiny = np.finfo(np.float32).tiny
+    assert ((want != 0) & (np.abs(want) < tiny)).mean() > 0.02 and (np.abs(want) >= tiny).mean() > 0.02
+    assert np.array_equal(got, want)
