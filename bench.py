@@ -77,19 +77,33 @@ def roofline_peaks(achieved):
                                  f"(copy: {pk['copy']} GB/s read+written)"}
 
 
+def kernel_sources():
+    """interp.hip and the csrc headers it includes, themselves or through
+    another: what the interpreter's kernels are compiled from."""
+    import re
+    d = os.path.join(ROOT, "sinter-qwen36-nomtp-tu102_amd", "csrc")
+    seen, todo = set(), ["interp.hip"]
+    while todo:
+        fn = todo.pop()
+        if fn in seen or not os.path.exists(os.path.join(d, fn)):
+            continue
+        seen.add(fn)
+        with open(os.path.join(d, fn)) as f:
+            todo += re.findall(r'^#include "([^"/]+)"', f.read(), re.M)
+    return [os.path.join(d, fn) for fn in sorted(seen)]
+
+
 def kernel_source_digest():
-    """sha256 of the interpreter's sources (interp.hip and the csrc/*.h
-    headers, sorted by name) and of the compiler flags it is built with
-    (build.py FLAGS): the traffic summary records the digest of the build it
-    was measured on.  Other translation units of the library (the batched
-    GEMV) do not enter it: they are separate code objects."""
+    """sha256 of the interpreter's sources (kernel_sources) and of the
+    compiler flags it is built with (build.py FLAGS): the traffic summary
+    records the digest of the build it was measured on.  Other translation
+    units of the library (the batched GEMV and prefill) and their headers do
+    not enter it: they are separate code objects."""
     import hashlib
     import importlib.util
     pkg = os.path.join(ROOT, "sinter-qwen36-nomtp-tu102_amd")
-    d = os.path.join(pkg, "csrc")
     h = hashlib.sha256()
-    files = [os.path.join(d, fn) for fn in sorted(os.listdir(d)) if fn.endswith(".h") or fn == "interp.hip"]
-    for path in files:
+    for path in kernel_sources():
         h.update(os.path.basename(path).encode())
         with open(path, "rb") as f:
             h.update(f.read())

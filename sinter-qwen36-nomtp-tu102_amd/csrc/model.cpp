@@ -34,6 +34,7 @@
 #include <utility>
 #include <vector>
 
+#include "batched.h"
 #include "internal.h"
 #include "synth.h"
 

@@ -19,6 +19,7 @@
 // logits are bit-identical to the decode program's.
 #include <algorithm>
 
+#include "batched.h"
 #include "internal.h"
 #include "gemv.h"
 #include "attn.h"

@@ -31,6 +31,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "batched.h"
 #include "internal.h"
 #include "dev_common.h"
 

@@ -45,3 +45,16 @@ def test_cpu_baseline_stops_at_the_last_kv_row(monkeypatch):
     m = types.SimpleNamespace(cfg=types.SimpleNamespace(n_ctx=4157))
     r = bench.cpu_baseline(m, 4096, 1e9)
     assert seen == list(range(4096, 4157)) and r["value"] > 0
+
+
+def test_traffic_depends_on_the_interpreters_own_sources_only():
+    """The figure is for what interp.hip is compiled from: a change to the
+    batched prefill's units or their header leaves it valid."""
+    names = {os.path.basename(p) for p in bench.kernel_sources()}
+    assert {"interp.hip", "internal.h", "isa.h", "dev_common.h", "gemv.h", "gdn.h", "attn.h", "synth.h"} == names
+    csrc = os.path.join(ROOT, "sinter-qwen36-nomtp-tu102_amd", "csrc")
+    others = [f for f in os.listdir(csrc) if f.endswith((".h", ".hip")) and f not in names]
+    assert "batched.h" in others and "ubatch.hip" in others
+    for f in names:
+        with open(os.path.join(csrc, f)) as s:
+            assert "batched.h" not in s.read(), f
