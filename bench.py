@@ -377,7 +377,7 @@ def ubatch_bench(args):
                    "per_matrix": per, "oracle_spot_check": check},
         "roofline": {"bound": "mfma", "achieved": round(tops, 1), "peak": MFMA_INT8_PEAK_TOPS, "unit": "TOP/s",
                      "frac": round(tops / MFMA_INT8_PEAK_TOPS, 4), "traffic": None,
-                     "kernel": "ubatch_gemv_kernel",
+                     "kernel": "ubatch_gemm_kernel (the many-token split), ubatch_gemv_kernel (the few-token one)",
                      "weights_gbs": round(layer_bytes / (ms * 1e-3) / 1e9, 1)},
     }
     if not args.no_cpu_baseline:

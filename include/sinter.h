@@ -296,8 +296,8 @@ int sinter_op_attn_decode(const sinter_attn_args *a, uint32_t blocks, void *stre
  * blocks of 292 bytes), for t < n_tokens: the single-token GEMV's fp64 item
  * terms folded in item order, so each y[t] is bit-identical to
  * sinter_op_gemv on token t alone.  accumulate != 0: y[t * rows + r] +=
- * the result instead (the RESID epilogue's residual add).  Weights are read
- * once per 64 tokens.
+ * the result instead (the RESID epilogue's residual add).  No byte past the
+ * last row or token is read.
  * Alignment: w 16 bytes (Q4_K) / 4 bytes (Q6_K), xq and y 4 bytes.
  * n_tokens == 0 is a no-op.  SINTER_ERR_ARG on a bad type, shape or
  * alignment (nothing launched). */

@@ -829,7 +829,8 @@ UbSplit ub_split_of(const UbArgs &a, UbSplit::Kernel kernel, uint32_t nt) {
 //   each further token's activations are another line of a load.
 // E.g. Q6_K 5120 x 17408 at 256 tokens (us): nt 2 180, 3 131, 4 143, 6 118,
 // 8 143; at 5 tokens few-token 37, many-token 90; 151936 x 5120 at 1, 5 and 16
-// tokens: few-token 154, 162, 193, many-token 175, 186, 195.  Q4_K 34816 x 5120 at 256:
+// tokens: few-token 154, 162, 193, many-token 175, 186, 195 (its price leaves
+// the tokens of a tile out: at 16 it is taken, 1 % over).  Q4_K 34816 x 5120 at 256:
 // nt 2 205, 4 180, 6 181, 8 166; 8192 x 5120 at 24: few-token 15, nt 1 15.5.
 // Short rows are mostly start-up, which these prices leave out: one item goes
 // to SHORT, two do where the few-token kernel would take them with more than

@@ -100,7 +100,7 @@ def test_prefill_refuses_bad_arguments(sn, torch_gpu):
 
 # (ubatch, KV type, attn_chunks, attn_chunk_min, context, prompt): one-token
 # ubatches; a ragged 7; chunks of 2 and 3 per kv head, where a query's chunk
-# length (tiles per chunk) changes every few positions, so the 8 queries of a
+# length (tiles per chunk) changes every few positions, so the 16 queries of a
 # block split differently; a Q8_0 cache
 BATCH_CASES = [
     (1, "f16", 0, 0, 0, 40),
