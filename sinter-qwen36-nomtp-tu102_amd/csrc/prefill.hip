@@ -103,7 +103,8 @@ __global__ __launch_bounds__(256) void gdn_prep_ubatch_kernel(GdnUb a) {
 // units (row order put them 64 bytes apart, four to a bank) -- and are read
 // into registers a token ahead; a stage belongs to one wave, so there is no
 // barrier.  27B shapes, 256 tokens: 139 us with four-wave workgroups, row
-// order and a barrier per stage, 80 us so.
+// order and a barrier per stage, 80 us so; with the prep kernel and 32 heads,
+// head size 64 99 -> 53, 128 147 -> 90, 256 229 -> 163 (one wave per SIMD).
 constexpr uint32_t GDN_STAGE = 8;
 static_assert(GDN_STAGE <= 8, "a stage's outputs fit the threads of a column");
 template <uint32_t RPT, uint32_t TPC>
@@ -372,15 +373,15 @@ static_assert(PF_Q8_VS + 32 * 8 * 4 <= PF_TILES, "Q8_0 tiles fit the tile region
 // Work item = (kv head g, split chunk c, q head hh of g's group, block of 16
 // consecutive queries), the block index running over the query blocks
 // first, so the items that read one chunk of one kv head run side by side.
-// Query i of the ubatch (position pos0 + i) is split exactly as the decode splits it at that position: att_geom(pos0 + i + 1,
-// C, chunk_min) chunks of tpc tiles, chunk c holding rows [c tpc 32,
-// min((c + 1) tpc 32, pos0 + i + 1)).  The item runs the union of its
-// queries' chunk-c rows in the decode attention's tiles; a row outside a
-// query's own range is masked out of its scores and enters its V sums as
-// fmaf(0, v, acc) (no change but the sign of a zero sum, which the Q8_K
-// quantisation of the attention output erases), or not at all where v is not
-// finite.  Per query the chunk partial
-// -- the 8 row groups merged, O, M, L -- is the decode's, bit for bit.
+// Query i of the ubatch (position pos0 + i) is split exactly as the decode
+// splits it at that position: att_geom(pos0 + i + 1, C, chunk_min) chunks of
+// tpc tiles, chunk c holding rows [c tpc 32, min((c + 1) tpc 32, pos0 + i +
+// 1)).  The item runs the union of its queries' chunk-c rows in the decode
+// attention's tiles; a row outside a query's own range is masked out of its
+// scores and enters its V sums as fmaf(0, v, acc) (no change but the sign of a
+// zero sum, which the Q8_K quantisation of the attention output erases), or
+// not at all where v is not finite.  Per query the chunk partial -- the 8 row
+// groups merged, O, M, L -- is the decode's, bit for bit.
 //
 // The decode's fmaf chains run on v_mfma_f32_16x16x1_4b_f32: four 16 x 16
 // blocks, one product each, every output a single fmaf (checked bit for bit,
@@ -400,7 +401,9 @@ static_assert(PF_Q8_VS + 32 * 8 * 4 <= PF_TILES, "Q8_0 tiles fit the tile region
 // tile's.  K rows lie in LDS as 16-byte chunks, chunk p at slot p ^ (row %
 // 16), so 16 rows' reads of one chunk hit distinct banks.  256 queries behind
 // 8192 positions, 27B shapes: 1.60 ms with VALU chains (8 queries per item),
-// 0.99 ms so.
+// 0.99 ms so.  An item costs the same for fewer queries, where the chains took
+// half the slots: 8 queries behind 8192 positions 75 and 73 us, behind 131,008
+// 630 and 715.
 template <bool Q8>
 __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(AttnPrefill a, uint32_t cmax) {
     __shared__ __attribute__((aligned(16))) unsigned char tiles[PF_TILES];
@@ -626,8 +629,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(AttnPrefill 
             // that is not finite is added here, to the queries that hold its
             // row, and is 0 below, where a zero weight would not keep it out of
             // the others.  (Selects and no branches inside, and out of the
-            // loop's way: 256 queries behind 8192 positions 968 -> 985 us; a
-            // branch per value 989, behind 131008 10.90 and 11.21 ms.)
+            // loop's way: 256 queries behind 8192 positions 968 us without,
+            // 985 so, 989 with a branch per value; behind 131,008 10.76, 10.90
+            // and 11.21 ms.)
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(partial) != 0, 0)) {
                 // (the lane is opaque: addresses made of it would be kept in
                 // registers through the loop, and spill)

@@ -359,11 +359,12 @@ def test_conv_silu_ubatch_token_edges(sn, orc, torch_gpu, dconv, n_tok):
     test_conv_silu_ubatch_matches_oracle_token_loop(sn, orc, torch_gpu, 300, dconv, n_tok)
 
 
-@pytest.mark.parametrize("k,n_tok", [(2048, 256), (2048, 257), (2048, 768), (2048, 769), (1792, 257), (8448, 300)])
-def test_rmsnorm_quant_q8k_ubatch_wave_rule(sn, orc, torch_gpu, k, n_tok):
+@pytest.mark.parametrize("k,n_tok,weighted", [(2048, 256, True), (2048, 257, True), (2048, 768, False), (2048, 769, True),
+                                              (1792, 257, False), (8448, 300, True)])
+def test_rmsnorm_quant_q8k_ubatch_wave_rule(sn, orc, torch_gpu, k, n_tok, weighted):
     """Both sides of the launch's lines: 16 waves a row up to 256 rows, 8 from
     8 blocks a row up to 96 rows per block, 4 past that."""
-    test_rmsnorm_quant_q8k_ubatch_matches_oracle(sn, orc, torch_gpu, k, n_tok, True)
+    test_rmsnorm_quant_q8k_ubatch_matches_oracle(sn, orc, torch_gpu, k, n_tok, weighted)
 
 
 def test_rmsnorm_quant_q8k_ubatch_many_rows(sn, torch_gpu):
